@@ -13,6 +13,8 @@
 //   * register-resident sweep (kron_reg.hpp) for the (d, n) plans listed in reg_plan(): the tensor lives
 //     in registers, n^RHO values per thread, with LDS only between phases; a workgroup walks a run of
 //     entries and accumulates same-output contributions in registers before one atomic flush;
+//   * block sweep (kron_block.hpp, kron_final.hpp) for the other shapes of the reference's grid above 200 elements:
+//     whole entries in LDS, larger vectors in one pass in LDS and one in registers;
 //   * fiber sweep (any d, n <= 64): the n^d vector lives in LDS (<= 64 KiB) or, beyond that, in the
 //     caller's per-entry workspace; one workgroup per entry; shared outputs are accumulated with
 //     hardware FP64/FP32 atomics (global_atomic_add_f64/f32).
@@ -29,6 +31,8 @@
 #include <vector>
 
 #include "kron_adjoint.hpp"
+#include "kron_block.hpp"
+#include "kron_final.hpp"
 #include "kron_group.hpp"
 #include "kron_mfma.hpp"
 #include "kron_ordered.hpp"
@@ -637,13 +641,121 @@ hipError_t wide_dispatch(Shape const &s, Launch &L, T const *const *mats, T cons
     return wide_launch<T, false>(s, L, chunk, mats, in, out, ws, stream, run);
 }
 
+// ---- block sweep (kron_block.hpp, kron_final.hpp): part of the fiber family, its default where a shape is built ----
+// Workgroups per CU: enough for about 12 (FP64) or 16 (FP32) wavefronts, at most 4. Fewer, longer runs save atomics,
+// more hide the entries' chains. Measured with 4608 entries and 5 outputs at 1 / 2 / 3 / 4 / 6 workgroups per CU: d=5
+// n=5 FP64 (10 wavefronts) 54 / 46 / 50 / 62 / 67 us; d=4 n=7 FP64 (6) 59 / 46 / 47 / 58 / 64, FP32 42 / 31 / 30 / 32
+// / 39; d=4 n=5 FP64 (2) 27 / 19 / 17 / 17 / 19; d=4 n=9 FP64 (12) 126 / 130 / 141 / 156 / 175.
+constexpr int block_workgroups_per_cu(int threads, int elem)
+{
+    int const waves = threads / 64, want = elem == 8 ? 12 : 16;
+    int const w = (want + waves - 1) / waves;
+    return w > 4 ? 4 : w;
+}
+
+template<typename T, int D, int N>
+hipError_t block_launch_dn(Shape const &s, Launch &L, T const *const *mats, T const *const *in, T *const *out,
+                           hipStream_t stream, bool run)
+{
+    constexpr int P = kronblock::block_threads<N, D>();
+    auto kernel = kronblock::kron_block_kernel<T, N, D, P>;
+    L.family = KRONMULT_FAMILY_FIBER;
+    L.block = P;
+    L.lds = sizeof(T) * kronblock::Block<T, N, D, 1, P>::LDS;
+    L.workspace = !fiber_in_lds<T>(s);  // a vector above the limit asks for one on every path
+    L.resident = resident_per_cu(kernel, P, 0);
+    long const slots = static_cast<long>(device_cu_count()) * block_workgroups_per_cu(P, sizeof(T));
+    L.epw = static_cast<int>((s.nb + slots - 1) / slots);
+    if (L.epw < 1) L.epw = 1;
+    long const runs = (static_cast<long>(s.nb) + L.epw - 1) / L.epw;
+    L.grid = (runs + 7) / 8 * 8;  // whole XCD stripes; surplus runs exit at once
+    if (!run) return hipSuccess;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(L.grid)), dim3(P), 0, stream, s.nb, L.epw, mats, s.stride, in,
+                       out);
+    return hipGetLastError();
+}
+
+template<typename T>
+hipError_t block_launch(Shape const &s, Launch &L, T const *const *mats, T const *const *in, T *const *out,
+                        hipStream_t stream, bool run)
+{
+#define KRON_BLOCK_LAUNCH(D, N) \
+    if constexpr (kronblock::block_shape<T>(D, N)) \
+        if (s.d == D && s.n == N) return block_launch_dn<T, D, N>(s, L, mats, in, out, stream, run);
+    KRON_BLOCK_SHAPES(KRON_BLOCK_LAUNCH)
+#undef KRON_BLOCK_LAUNCH
+    return hipErrorInvalidValue;
+}
+
+// d = D: the block pass over the D - 2 fastest modes into the workspace, then modes 1 and 0 from there
+template<typename T, int D, int N>
+hipError_t block_passes_dn(Shape const &s, Launch &L, T const *const *mats, T const *const *in, T *const *out,
+                           T *const *ws, hipStream_t stream, bool run)
+{
+    constexpr int G = D - 2, P = kronblock::pass_threads<T, N>(), Q = kronblock::ipow(N, 4 - G);
+    constexpr int RB = kronfinal::rows<T, N>();
+    using B = kronblock::Block<T, N, G, Q, P>;
+    constexpr int kInner = kronblock::ipow(N, G);
+    constexpr int kPerEntry = kronblock::ipow(N, D) / B::S;
+    constexpr int kTiles = (kInner + kronfinal::kLanes - 1) / kronfinal::kLanes;
+    long const cus = device_cu_count();
+    long const items = static_cast<long>(s.nb) * kPerEntry;
+    long block_run = 1;
+    if (P > kronblock::kPassOneBlockThreads)
+        block_run = std::max(1l, (items + cus * kronblock::kPassWorkgroupsPerCu - 1) / (cus * kronblock::kPassWorkgroupsPerCu));
+    long const block_grid = ((items + block_run - 1) / block_run + 7) / 8 * 8;
+    // entries per wavefront of the second pass
+    long const waves = static_cast<long>(kTiles) * (N / RB) * s.nb;
+    long const final_run = std::min<long>(kronfinal::kMaxRun, std::max(1l, waves / (cus * kronfinal::kWavesPerCu)));
+    long const groups = (s.nb + final_run * kronfinal::kWaves - 1) / (final_run * kronfinal::kWaves);
+    long const final_grid = (groups * kTiles * (N / RB) + 7) / 8 * 8;
+    L.family = KRONMULT_FAMILY_FIBER;
+    L.block = P;
+    L.epw = 1;
+    L.grid = block_grid;
+    L.lds = sizeof(T) * B::LDS;
+    L.workspace = true;
+    if (items > INT_MAX - 8 || final_grid > INT_MAX) return hipErrorInvalidValue;
+    auto pass = kronblock::kron_block_pass_kernel<T, N, G, Q, P>;
+    auto last = kronfinal::kron_final_kernel<T, N, RB>;
+    L.resident = resident_per_cu(pass, P, 0);
+    if (!run) return hipSuccess;
+    hipLaunchKernelGGL(pass, dim3(static_cast<unsigned>(block_grid)), dim3(P), 0, stream, static_cast<int>(items),
+                       kPerEntry, static_cast<int>(block_run), D, mats, s.stride, in, ws);
+    hipError_t const err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    hipLaunchKernelGGL(last, dim3(static_cast<unsigned>(final_grid)), dim3(kronfinal::kLanes * kronfinal::kWaves), 0,
+                       stream, s.nb, static_cast<int>(final_run), kTiles, kInner, D, mats, s.stride,
+                       reinterpret_cast<T const *const *>(ws), out);
+    return hipGetLastError();
+}
+
+template<typename T>
+hipError_t block_passes(Shape const &s, Launch &L, T const *const *mats, T const *const *in, T *const *out,
+                        T *const *ws, hipStream_t stream, bool run)
+{
+#define KRON_PASS_LAUNCH(D, N) \
+    if constexpr (kronblock::pass_shape<T>(D, N)) \
+        if (s.d == D && s.n == N) return block_passes_dn<T, D, N>(s, L, mats, in, out, ws, stream, run);
+    KRON_PASS_LAUNCH(5, 7) KRON_PASS_LAUNCH(5, 8) KRON_PASS_LAUNCH(5, 9) KRON_PASS_LAUNCH(5, 10)
+    KRON_PASS_LAUNCH(6, 5) KRON_PASS_LAUNCH(6, 6) KRON_PASS_LAUNCH(6, 7) KRON_PASS_LAUNCH(6, 8)
+    KRON_PASS_LAUNCH(6, 9) KRON_PASS_LAUNCH(6, 10)
+#undef KRON_PASS_LAUNCH
+    return hipErrorInvalidValue;
+}
+
 template<typename T>
 hipError_t fiber_dispatch(Shape const &s, Launch &L, T const *const *mats, T const *const *in, T *const *out,
                           T *const *ws, hipStream_t stream, bool run)
 {
     if (s.n > kMaxFiber) return wide_dispatch<T>(s, L, mats, in, out, ws, stream, run);
-    if (fiber_in_lds<T>(s)) return fiber_dispatch_n<T, true>(s, L, mats, in, out, ws, stream, run);
+    bool const block = !s.ordered && kronblock::block_shape<T>(s.d, s.n);
+    if (fiber_in_lds<T>(s))
+        return block ? block_launch<T>(s, L, mats, in, out, stream, run)
+                     : fiber_dispatch_n<T, true>(s, L, mats, in, out, ws, stream, run);
     if (run && ws == nullptr) return hipErrorInvalidValue;
+    if (block) return block_launch<T>(s, L, mats, in, out, stream, run);
+    if (!s.ordered && kronblock::pass_shape<T>(s.d, s.n)) return block_passes<T>(s, L, mats, in, out, ws, stream, run);
     if (use_passes<T>(s)) return pass_dispatch<T>(s, L, mats, in, out, ws, stream, run);
     return fiber_dispatch_n<T, false>(s, L, mats, in, out, ws, stream, run);
 }

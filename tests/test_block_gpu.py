@@ -1,0 +1,72 @@
+"""GPU parity of the block sweep (whole entries in LDS, and the block pass plus the register pass of larger vectors)
+with the oracle: bit for bit where each output has one contribution, within the accumulation bound where outputs are
+shared. Runs are cut inside and between outputs, strides are padded and odd entries' inputs only element-aligned."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import accumulation_bound, grouped_by_output, normwise, shift_odd_inputs
+from kronmult993_amd import api, workloads as W
+from kronmult993_amd.device import DeviceBatch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [np.float64, np.float32]
+EPS = {np.dtype(np.float64): np.finfo(np.float64).eps / 2, np.dtype(np.float32): np.finfo(np.float32).eps / 2}
+
+
+def _run(b, gpu):
+    print(f"[case] {b.name} d={b.d} n={b.n} nb={b.nb} {b.dtype}", flush=True)
+    db = DeviceBatch(b, device=str(gpu), workspace="per_entry")
+    inputs = db.inp.clone()
+    db.run()
+    assert bool((db.inp == inputs).all())
+    return db.output()
+
+
+def _check(b, gpu):
+    u = W.HostBatch(**{**b.__dict__, "out_count": b.nb, "out_index": np.arange(b.nb, dtype=np.int64), "out_init": None})
+    assert np.array_equal(_run(u, gpu), oracle.kronmult(u))
+    for case in (b, grouped_by_output(b)):
+        err = np.abs(_run(case, gpu).astype(np.float64) - oracle.kronmult(case).astype(np.float64))
+        assert float(np.max(err - accumulation_bound(case, EPS[case.dtype]))) <= 0.0
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("d,n", [(3, 6), (3, 7), (3, 9), (3, 10), (4, 5), (4, 6), (4, 7), (4, 9), (4, 10), (5, 5),
+                                 (5, 6), (6, 3), (6, 5)])
+def test_whole_entries(gpu, d, n, dtype):
+    assert api.kernel_name(d, n, np.dtype(dtype).itemsize, 50).startswith(("fiber", "wave", "multipass"))
+    _check(shift_odd_inputs(W.random_case(310 + 7 * d + n, d, n, 50, stride=n + d % 3, shared_factors=17, dtype=dtype)),
+           gpu)
+
+
+@pytest.mark.parametrize("d,n,dtype,nb", [(3, 6, np.float64, 2600), (4, 5, np.float64, 1700), (4, 7, np.float32, 1300),
+                                          (5, 5, np.float64, 1100), (4, 9, np.float64, 600), (6, 3, np.float32, 2500)])
+def test_runs_of_entries(gpu, d, n, dtype, nb):
+    """More entries than resident workgroups: runs of two and more entries, a shorter last one."""
+    _check(W.random_case(330 + d + n, d, n, nb, stride=n + 1, shared_factors=211, distinct=nb // 4 + 1, dtype=dtype), gpu)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("d,n", [(5, 7), (5, 8), (5, 9), (5, 10), (6, 5), (6, 6), (6, 7), (6, 8), (6, 9), (6, 10)])
+def test_large_vectors(gpu, d, n, dtype):
+    """Two passes; 9 entries of 3 outputs leave the four wavefronts of a workgroup on one output or on several."""
+    nb = 9 if n ** d <= 300000 else 5
+    _check(shift_odd_inputs(W.random_case(350 + 7 * d + n, d, n, nb, stride=n + n % 3, shared_factors=3, distinct=3,
+                                          dtype=dtype)), gpu)
+
+
+def test_large_vectors_run_lengths(gpu):
+    """Enough entries for runs of several per wavefront and of several blocks per workgroup (d=5 n=9 and d=5 n=7)."""
+    _check(W.random_case(371, 5, 7, 1500, shared_factors=40, distinct=7, dtype=np.float32), gpu)
+    _check(W.random_case(372, 5, 9, 300, shared_factors=40, distinct=5, dtype=np.float64), gpu)
+
+
+@pytest.mark.parametrize("d,n,itemsize", [(4, 10, 8), (5, 7, 8), (6, 5, 8), (6, 10, 4)])
+def test_large_vectors_need_a_workspace(gpu, d, n, itemsize):
+    dtype = np.float64 if itemsize == 8 else np.float32
+    assert api.launch_info(d, n, itemsize, 2)["uses_workspace"] == 1
+    db = DeviceBatch(W.random_case(380, d, n, 2, dtype=dtype), device=str(gpu), workspace="none")
+    with pytest.raises(api.KronmultError):
+        db.run()
