@@ -338,7 +338,7 @@ __global__ void __launch_bounds__(P)
 // Whole entries, as X(D, N): the (d, n) of the reference's grid (d <= 6, n <= 10) whose vector stays on chip and
 // that no other kernel takes by default.
 #define KRON_BLOCK_SHAPES(X)                                                                                        \
-    X(3, 6) X(3, 7) X(3, 9) X(3, 10) X(4, 5) X(4, 6) X(4, 7) X(4, 9) X(4, 10) X(5, 5) X(5, 6) X(6, 3) X(6, 5)
+    X(3, 9) X(3, 10) X(4, 6) X(4, 7) X(4, 9) X(4, 10) X(5, 5) X(5, 6) X(6, 3) X(6, 5)
 // d=6 n=5 FP64 (125 KB) and d=4 n=10 FP64 (80 KB) take a workspace like every vector above 64 KB; the second
 // still fits a workgroup's LDS, with one workgroup of 16 wavefronts per CU.
 template<typename T>

@@ -189,10 +189,10 @@ __global__ void __launch_bounds__(kLanes)
 #define KRON_WAVE_SHAPES(X)                                                                                      \
     X(1, 2) X(2, 2) X(3, 2) X(4, 2) X(5, 2) X(6, 2) X(1, 3) X(2, 3) X(3, 3) X(1, 4) X(2, 4) X(3, 4) X(1, 5)       \
         X(2, 5) X(1, 6) X(2, 6) X(1, 7) X(2, 7) X(1, 8) X(2, 8)
-// Shapes with 2 to 4 elements per lane and no register-resident plan (single batch only).
-#define KRON_WAVE_SHAPES_WIDE(X) X(7, 2) X(8, 2) X(4, 3) X(5, 3) X(3, 5) X(3, 6) X(2, 9) X(2, 10)
+// Shapes with two elements per lane (single batch only; kron_wave_fiber.hpp takes the other ones of the family).
+#define KRON_WAVE_SHAPES_WIDE(X) X(3, 5) X(2, 9) X(2, 10)
 
-// whether (d, n) is one of the shapes above
+// the shapes of the wave family: the ones above, and from kron_wave_fiber.hpp (7,2) (8,2) (4,3) (5,3) (3,6)
 __host__ __device__ constexpr bool wave_family_shape(int d, int n)
 {
     if (wave_shape(d, n)) return true;

@@ -42,6 +42,7 @@
 #include "kron_reg.hpp"
 #include "kron_m8.hpp"
 #include "kron_wave.hpp"
+#include "kron_wave_fiber.hpp"
 #include "kron_reg_adjoint.hpp"
 #include "kron_reg_adjoint2.hpp"
 #include "kronmult_hip.h"
@@ -641,11 +642,45 @@ hipError_t wide_dispatch(Shape const &s, Launch &L, T const *const *mats, T cons
     return wide_launch<T, false>(s, L, chunk, mats, in, out, ws, stream, run);
 }
 
+// ---- one wavefront per entry, whole fibers per lane (kron_wave_fiber.hpp) ---------------------------------
+// Default run of a wavefront: two entries once the batch gives every CU 16 wavefronts with one (6000 entries of d=3
+// n=6 FP64, four per output: 8.1 / 8.0 / 8.5 / 9.6 us with runs of 1 / 2 / 3 / 4; 4608 with 5 outputs 11.4 / 8.3 / 8.3 /
+// 9.7), else one (1500 of d=5 n=3: 4.4 / 4.7 / 5.7 / 6.6).
+constexpr long kWaveFiberEntriesPerCu = 16;
+
+template<typename T>
+hipError_t wave_fiber_launch(Shape const &s, int family, int entries_per_workgroup, Launch &L, T const *const *mats,
+                             T const *const *in, T *const *out, hipStream_t stream, bool run)
+{
+    int epw = s.nb > kWaveFiberEntriesPerCu * device_cu_count() ? 2 : 1;
+    if (entries_per_workgroup > 0) epw = (std::min(entries_per_workgroup, s.nb) - 1) / kronwave::kWaves + 1;
+    if (epw < 1) epw = 1;
+    L.family = family;
+    L.block = kronwave::kLanes * kronwave::kWaves;
+    long const per_wg = static_cast<long>(epw) * kronwave::kWaves;
+    L.epw = static_cast<int>(std::min<long>(per_wg, INT_MAX));
+    L.grid = ((s.nb + per_wg - 1) / per_wg + 7) / 8 * 8;  // whole XCD stripes; surplus workgroups exit at once
+#define KRON_WAVE_FIBER_LAUNCH(D, N)                                                                                   \
+    if (s.d == D && s.n == N)                                                                                          \
+    {                                                                                                                  \
+        auto kernel = kronwave::kron_wave_fiber_kernel<T, D, N>;                                                       \
+        L.lds = sizeof(T) * kronwave::kWaves * kronwave::FiberWave<T, D, N>::LDS;                                      \
+        L.resident = resident_per_cu(kernel, L.block, 0);                                                              \
+        if (!run || s.nb == 0) return hipSuccess;                                                                      \
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(L.grid)), dim3(L.block), 0, stream, s.nb, epw, mats,     \
+                           s.stride, in, out);                                                                         \
+        return hipGetLastError();                                                                                      \
+    }
+    KRON_WAVE_FIBER_SHAPES(KRON_WAVE_FIBER_LAUNCH)
+#undef KRON_WAVE_FIBER_LAUNCH
+    return hipErrorInvalidValue;
+}
+
 // ---- block sweep (kron_block.hpp, kron_final.hpp): part of the fiber family, its default where a shape is built ----
 // Workgroups per CU: enough for about 12 (FP64) or 16 (FP32) wavefronts, at most 4. Fewer, longer runs save atomics,
 // more hide the entries' chains. Measured with 4608 entries and 5 outputs at 1 / 2 / 3 / 4 / 6 workgroups per CU: d=5
 // n=5 FP64 (10 wavefronts) 54 / 46 / 50 / 62 / 67 us; d=4 n=7 FP64 (6) 59 / 46 / 47 / 58 / 64, FP32 42 / 31 / 30 / 32
-// / 39; d=4 n=5 FP64 (2) 27 / 19 / 17 / 17 / 19; d=4 n=9 FP64 (12) 126 / 130 / 141 / 156 / 175.
+// / 39; d=4 n=6 FP64 (4) 42 / 29 / 27 / 27 / 32; d=4 n=9 FP64 (12) 126 / 130 / 141 / 156 / 175.
 constexpr int block_workgroups_per_cu(int threads, int elem)
 {
     int const waves = threads / 64, want = elem == 8 ? 12 : 16;
@@ -749,6 +784,9 @@ hipError_t fiber_dispatch(Shape const &s, Launch &L, T const *const *mats, T con
                           T *const *ws, hipStream_t stream, bool run)
 {
     if (s.n > kMaxFiber) return wide_dispatch<T>(s, L, mats, in, out, ws, stream, run);
+    // (4,3), (5,3), (7,2) and (8,2) come here only when a caller asks for this family: the general kernel
+    if (!s.ordered && ((s.d == 3 && (s.n == 6 || s.n == 7)) || (s.d == 4 && s.n == 5)))
+        return wave_fiber_launch<T>(s, KRONMULT_FAMILY_FIBER, 0, L, mats, in, out, stream, run);
     bool const block = !s.ordered && kronblock::block_shape<T>(s.d, s.n);
     if (fiber_in_lds<T>(s))
         return block ? block_launch<T>(s, L, mats, in, out, stream, run)
@@ -832,6 +870,8 @@ template<typename T>
 hipError_t packed_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L, T const *const *mats,
                          T const *const *in, T *const *out, hipStream_t stream, bool run)
 {
+    if (tu.entries_per_workgroup == 0 && tu.workgroups_per_cu == 0 && kronwave::wave_fiber_shape(s.d, s.n))
+        return wave_fiber_launch<T>(s, KRONMULT_FAMILY_PACKED, 0, L, mats, in, out, stream, run);
     krongroup::GroupTable<T> table{};
     long const per_entry = group_entry_bytes<T>(s);
     int ept = tu.entries_per_workgroup;
@@ -870,9 +910,8 @@ hipError_t packed_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L,
 // 2.7 (fiber 3.5). Longer runs gave fewer workgroups than the latency needs, shorter ones more atomics.
 constexpr long kWaveRunsPerCu = 8;
 constexpr int kWaveMaxRun = 4;
-// 2 to 4 elements per lane: 20000 entries of d=7 n=2 13.6 us (packed launch 27.1), d=8 n=2 27.5 (fiber 44.0),
-// d=5 n=3 24.7 (fiber 47.3), d=4 n=3 10.7 (packed 13.5), d=3 n=5 14.2 (packed 17.4), d=3 n=6 29.3 (packed
-// 29.7) at runs of 2; runs of 4 were 1-7% slower, runs of 1 10-50% slower.
+// Two elements per lane: 20000 entries of d=3 n=5 14.2 us (packed launch 17.4) at runs of 2; runs of 4 were 1-7%
+// slower, runs of 1 10-50% slower.
 constexpr int kWaveMaxRunWide = 2;
 
 template<typename T, int D, int N>
@@ -914,7 +953,12 @@ hipError_t wave_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L, T
     KRON_WAVE_SHAPES(KRON_WAVE_LAUNCH)
     KRON_WAVE_SHAPES_WIDE(KRON_WAVE_LAUNCH)
 #undef KRON_WAVE_LAUNCH
-    return hipErrorInvalidValue;
+    if (!kronwave::wave_fiber_shape(s.d, s.n)) return hipErrorInvalidValue;
+    // a grid size asked for instead of a run length: the run that gives it
+    long const wgs = static_cast<long>(device_cu_count()) * tu.workgroups_per_cu;
+    int const epw = tu.entries_per_workgroup > 0 || wgs == 0 ? tu.entries_per_workgroup
+                                                              : static_cast<int>((s.nb + wgs - 1) / wgs);
+    return wave_fiber_launch<T>(s, KRONMULT_FAMILY_WAVE, epw, L, mats, in, out, stream, run);
 }
 
 // ---- entry --------------------------------------------------------------------------------------------
@@ -931,7 +975,7 @@ int choose_family(Shape const &s, kronmult_tuning_t const &tu)
     if (tu.family == KRONMULT_FAMILY_WAVE) return kronwave::wave_family_shape(s.d, s.n) ? KRONMULT_FAMILY_WAVE : -1;
     if (tu.family != KRONMULT_FAMILY_AUTO) return -1;
     if (reg_ok) return KRONMULT_FAMILY_REGISTER;
-    // d=3 n=6 FP64 (4 elements per lane, 152 VGPRs) measured 3-4% behind the packed launch
+    // d=3 n=6 FP64 belongs to the fiber and packed families by default; the kernel is the same in all three
     bool const wave_default = kronwave::wave_family_shape(s.d, s.n) && !(sizeof(T) == 8 && s.d == 3 && s.n == 6);
     if (wave_default) return KRONMULT_FAMILY_WAVE;
     if (packed_ok<T>(s) && s.nb >= kPackedEntriesPerCu * device_cu_count()) return KRONMULT_FAMILY_PACKED;

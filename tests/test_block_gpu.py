@@ -57,6 +57,31 @@ def test_large_vectors(gpu, d, n, dtype):
                                           dtype=dtype)), gpu)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("d,n", [(4, 3), (5, 3), (7, 2), (8, 2), (3, 6), (3, 7), (4, 5)])
+def test_whole_fibers_per_lane(gpu, d, n, dtype):
+    """One wavefront per entry: fewer entries than a workgroup's wavefronts, one per wavefront and two, the last
+    workgroup partly without entries; wavefronts of a workgroup on one output and on several."""
+    for nb in (3, 101, 4403):
+        _check(shift_odd_inputs(W.random_case(360 + 7 * d + n, d, n, nb, stride=n + d % 3, shared_factors=57,
+                                              distinct=nb // 6 + 1, dtype=dtype)), gpu)
+
+
+@pytest.mark.parametrize("family", [api.FAMILY_WAVE, api.FAMILY_FIBER, api.FAMILY_PACKED])
+def test_whole_fibers_per_lane_families(gpu, family):
+    """d=3 n=6 through each family that it belongs to, with run lengths and grids asked for."""
+    b = W.random_case(377, 3, 6, 333, distinct=40)
+    u = W.HostBatch(**{**b.__dict__, "out_count": b.nb, "out_index": np.arange(b.nb, dtype=np.int64), "out_init": None})
+    ref = oracle.kronmult(u)
+    for epw, wpc in ((0, 0), (1, 0), (7, 0), (2000000000, 0), (0, 1)):
+        tu = {"family": family, "entries_per_workgroup": epw, "workgroups_per_cu": wpc}
+        if family == api.FAMILY_PACKED and epw > 1000:
+            continue
+        db = DeviceBatch(u, device=str(gpu))
+        db.run(tuning=tu)
+        assert np.array_equal(db.output(), ref), tu
+
+
 def test_large_vectors_run_lengths(gpu):
     """Enough entries for runs of several per wavefront and of several blocks per workgroup (d=5 n=9 and d=5 n=7)."""
     _check(W.random_case(371, 5, 7, 1500, shared_factors=40, distinct=7, dtype=np.float32), gpu)
