@@ -244,12 +244,14 @@ long long kronmult_batched_adjoint_workspace(int matrix_count, int matrix_size, 
  * Strategies (options->strategy; options may be NULL = AUTO with defaults):
  *   KRONMULT_GROUPED_PERSISTENT  one persistent launch over every group with n <= 8 whose vector and
  *                                factors fit in 64 KiB of LDS; `workgroups_per_cu` sizes its grid (0 =
- *                                default 2) and each group's `entries_per_tile` its tiles (0 = one pass of
+ *                                default 8) and each group's `entries_per_tile` its tiles (0 = one pass of
  *                                min(256 / n^(d-1), what fits) entries; a shorter tile also shortens the pass,
- *                                which lowers the LDS per workgroup);
+ *                                which lowers the LDS per workgroup; groups swept one wavefront per entry take
+ *                                a quarter of the tile per wavefront, by default 4 entries, 2 above 64 elements);
  *                                any other group gets a launch of its own, as below;
  *   KRONMULT_GROUPED_SEPARATE    one ordinary launch per group, shaped by that group's `tuning`;
- *   KRONMULT_GROUPED_AUTO        currently the persistent strategy.
+ *   KRONMULT_GROUPED_AUTO        the persistent strategy, with launches of their own for large groups that a
+ *                                single-batch kernel sweeps faster.
  * Only the first 16 groups can take part in the persistent launch; later groups get launches of their own.
  */
 #define KRONMULT_GROUPED_AUTO 0

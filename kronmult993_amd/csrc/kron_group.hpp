@@ -11,12 +11,19 @@
 // entry to the reference's sweep with fused multiply-adds), and the results are added to the outputs:
 // consecutive entries of the pass that target the same output are summed in LDS order first, then one
 // hardware atomic add per element and run.
+//
+// Groups of small tensors skip the passes: each of the four wavefronts sweeps a quarter of the tile, one entry at a time
+// (kron_wave.hpp up to 64 elements, kron_wave_fiber.hpp for the larger shapes below), without workgroup barriers. The
+// passes wait on their staging loads and on six barriers per entry group: the mixed d=2..6 workload (31,300 entries,
+// default grid and tiles) went from 50 to 22.3 us FP64 and from 45 to 17.1 us FP32 with d=3 n=6, d=4 n=4 and d=5 n=3 on
+// the second path and 8 workgroups per CU instead of 2; it moves 74 MB, 15 us at the rate of a large copy.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include "kron_reg.hpp"
 #include "kron_wave.hpp"
+#include "kron_wave_fiber.hpp"
 
 namespace krongroup
 {
@@ -31,10 +38,41 @@ __host__ __device__ constexpr int wave_lds_elems()
     return kronwave::kLanes + kronwave::kMaxCoef;  // one element per lane, d n^2 <= 128
 }
 
+// How a group's tiles are swept: by the whole workgroup in passes (below), or by its wavefronts one entry each, a
+// lane per element (n^d <= 64, kron_wave.hpp) or with whole fibers per lane (kron_wave_fiber.hpp).
+constexpr int kPass = 0, kWave = 1, kWaveFiber = 2;
+
+// The shapes of the last path. FP64 leaves out d=3 n=7 and d=4 n=5: their 172 and 156 registers would spill under the
+// kernel's cap.
+#define KRON_GROUP_FIBER_SHAPES(X) X(3, 5) X(3, 6) X(3, 7) X(4, 3) X(4, 4) X(4, 5) X(5, 3) X(7, 2) X(8, 2)
+
+template<typename T>
+constexpr bool group_fiber_shape(int d, int n)
+{
+    if (sizeof(T) == 8 && ((d == 3 && n == 7) || (d == 4 && n == 5))) return false;
+#define KRON_GROUP_FIBER_IS(D, N) \
+    if (d == D && n == N) return true;
+    KRON_GROUP_FIBER_SHAPES(KRON_GROUP_FIBER_IS)
+#undef KRON_GROUP_FIBER_IS
+    return false;
+}
+
+// LDS elements of a workgroup for such a group, 0 for another shape
+template<typename T>
+constexpr int group_fiber_lds(int d, int n)
+{
+    if (!group_fiber_shape<T>(d, n)) return 0;
+#define KRON_GROUP_FIBER_LDS(D, N) \
+    if (d == D && n == N) return kronwave::kWaves * kronwave::FiberWave<T, D, N>::LDS;
+    KRON_GROUP_FIBER_SHAPES(KRON_GROUP_FIBER_LDS)
+#undef KRON_GROUP_FIBER_LDS
+    return 0;
+}
+
 template<typename T>
 struct GroupDesc
 {
-    int wave;  // 1: the group's tiles run on the wave path (n^d <= 64, kron_wave.hpp)
+    int path;  // kPass, kWave or kWaveFiber
     int d, n, stride, nb;
     int size;       // n^d
     int nfib;       // n^(d-1)
@@ -44,6 +82,15 @@ struct GroupDesc
     T const *const *in;
     T *const *out;
 };
+
+// A tile of a whole-fiber group
+template<typename T, int D, int N>
+__device__ __forceinline__ void fiber_tile(GroupDesc<T> const &G, int e0, int e1, int epw, T *lds, T **last, int wave,
+                                           int lane)
+{
+    if constexpr (group_fiber_shape<T>(D, N))
+        kronwave::FiberWave<T, D, N>::group(e0, e1, epw, G.mats, G.stride, G.in, G.out, lds, last, wave, lane);
+}
 
 template<typename T>
 struct GroupTable
@@ -155,11 +202,16 @@ __device__ __forceinline__ void pass(GroupDesc<T> const &G, int e0, int cnt, T *
     __syncthreads();  // LDS free for the next pass
 }
 
-// WAVE: the table may hold wave groups (the grouped launch). Their inlined paths take the kernel from 48 to
-// 82 VGPRs; the cap keeps 6 waves per SIMD without spills. The packed single-batch launch has no wave
-// groups and keeps 8 waves per SIMD.
-template<typename T, bool WAVE>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(WAVE ? 6 : 1)))
+// Waves per SIMD asked of the register allocator: 6 for passes and one-element wave groups together (80 VGPRs, no
+// spills), 5 with whole-fiber groups (96, none; at 4 the mixed workload takes 24.4 us against 22.3, at 6 it spills).
+constexpr int paths_waves_per_simd(int paths)
+{
+    return (paths & (1 << kWaveFiber)) != 0 ? 5 : (paths & (1 << kWave)) != 0 ? 6 : 1;
+}
+
+// PATHS: the paths that the table's groups may take (bit 1 << path).
+template<typename T, int PATHS>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(paths_waves_per_simd(PATHS))))
     kron_group_kernel(GroupTable<T> const table)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -172,30 +224,48 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W
         GroupDesc<T> const &G = table.g[gi];
         int const e_begin = (tile - table.tile_start[gi]) * G.epw;
         int const e_end = e_begin + G.epw < G.nb ? e_begin + G.epw : G.nb;
-        if (WAVE && G.wave)
-        {
-            // n^d <= 64: each wavefront sweeps a contiguous quarter of the tile on its own (kron_wave.hpp)
-            int const w = static_cast<int>(threadIdx.x) / kronwave::kLanes;
-            int const lane = static_cast<int>(threadIdx.x) - w * kronwave::kLanes;
-            int const chunk = (e_end - e_begin + kWaves - 1) / kWaves;
-            int const a = e_begin + w * chunk;
-            int const b = a + chunk < e_end ? a + chunk : e_end;
-            T *const xs = lds + w * wave_lds_elems();
-            T *const cs = xs + kronwave::kLanes;
-            if (a < b)
+        // wave paths: each wavefront sweeps a contiguous quarter of the tile on its own
+        int const w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kronwave::kLanes);
+        int const lane = static_cast<int>(threadIdx.x) & (kronwave::kLanes - 1);
+        int const chunk = (e_end - e_begin + kWaves - 1) / kWaves;
+        if constexpr ((PATHS & (1 << kWaveFiber)) != 0)
+            if (G.path == kWaveFiber)
             {
+                int lane_op = lane;
+                asm volatile("" : "+v"(lane_op));
                 switch (G.d * 16 + G.n)
                 {
-#define KRON_GROUP_WAVE(D, N)                                                                          \
-    case D * 16 + N: kronwave::wave_run<T, D, N, true>(a, b, G.mats, G.stride, G.in, G.out, xs, cs, lane); break;
-                    KRON_WAVE_SHAPES(KRON_GROUP_WAVE)
-#undef KRON_GROUP_WAVE
+#define KRON_GROUP_FIBER(D, N)                                                                                      \
+    case D * 16 + N: fiber_tile<T, D, N>(G, e_begin, e_end, chunk, lds, out_slot, w, lane_op); break;
+                    KRON_GROUP_FIBER_SHAPES(KRON_GROUP_FIBER)
+#undef KRON_GROUP_FIBER
                 default: break;
                 }
+                __syncthreads();  // LDS free for the next tile
+                continue;
             }
-            __syncthreads();  // LDS free for the next tile
-            continue;
-        }
+        if constexpr ((PATHS & (1 << kWave)) != 0)
+            if (G.path == kWave)
+            {
+                int const a = e_begin + w * chunk;
+                int const b = a + chunk < e_end ? a + chunk : e_end;
+                T *const xs = lds + w * wave_lds_elems();
+                T *const cs = xs + kronwave::kLanes;
+                if (a < b)
+                {
+                    switch (G.d * 16 + G.n)
+                    {
+#define KRON_GROUP_WAVE(D, N)                                                                          \
+    case D * 16 + N: kronwave::wave_run<T, D, N, true>(a, b, G.mats, G.stride, G.in, G.out, xs, cs, lane); break;
+                        KRON_WAVE_SHAPES(KRON_GROUP_WAVE)
+#undef KRON_GROUP_WAVE
+                    default: break;
+                    }
+                }
+                __syncthreads();  // LDS free for the next tile
+                continue;
+            }
+        if constexpr ((PATHS & (1 << kPass)) != 0)
         for (int e0 = e_begin; e0 < e_end; e0 += G.E)
         {
             int const cnt = e_end - e0 < G.E ? e_end - e0 : G.E;

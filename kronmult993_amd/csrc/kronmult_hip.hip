@@ -665,7 +665,7 @@ hipError_t wave_fiber_launch(Shape const &s, int family, int entries_per_workgro
     {                                                                                                                  \
         auto kernel = kronwave::kron_wave_fiber_kernel<T, D, N>;                                                       \
         L.lds = sizeof(T) * kronwave::kWaves * kronwave::FiberWave<T, D, N>::LDS;                                      \
-        L.resident = resident_per_cu(kernel, L.block, 0);                                                              \
+        if (!run) L.resident = resident_per_cu(kernel, L.block, 0);                                                    \
         if (!run || s.nb == 0) return hipSuccess;                                                                      \
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(L.grid)), dim3(L.block), 0, stream, s.nb, epw, mats,     \
                            s.stride, in, out);                                                                         \
@@ -698,7 +698,7 @@ hipError_t block_launch_dn(Shape const &s, Launch &L, T const *const *mats, T co
     L.block = P;
     L.lds = sizeof(T) * kronblock::Block<T, N, D, 1, P>::LDS;
     L.workspace = !fiber_in_lds<T>(s);  // a vector above the limit asks for one on every path
-    L.resident = resident_per_cu(kernel, P, 0);
+    if (!run) L.resident = resident_per_cu(kernel, P, 0);
     long const slots = static_cast<long>(device_cu_count()) * block_workgroups_per_cu(P, sizeof(T));
     L.epw = static_cast<int>((s.nb + slots - 1) / slots);
     if (L.epw < 1) L.epw = 1;
@@ -753,7 +753,7 @@ hipError_t block_passes_dn(Shape const &s, Launch &L, T const *const *mats, T co
     if (items > INT_MAX - 8 || final_grid > INT_MAX) return hipErrorInvalidValue;
     auto pass = kronblock::kron_block_pass_kernel<T, N, G, Q, P>;
     auto last = kronfinal::kron_final_kernel<T, N, RB>;
-    L.resident = resident_per_cu(pass, P, 0);
+    if (!run) L.resident = resident_per_cu(pass, P, 0);
     if (!run) return hipSuccess;
     hipLaunchKernelGGL(pass, dim3(static_cast<unsigned>(block_grid)), dim3(P), 0, stream, static_cast<int>(items),
                        kPerEntry, static_cast<int>(block_run), D, mats, s.stride, in, ws);
@@ -816,12 +816,23 @@ bool group_persistent_ok(GroupT const &g, Shape const &s)
     return s.n <= 8 && group_entry_bytes<T>(s) <= static_cast<long>(kGroupLdsBudget);
 }
 
-// One group's descriptor; returns the LDS bytes its passes take.
+// Default grid and tiles of the grouped launch. Measured on the mixed d=2..6 workload (31,300 entries, FP64 / FP32) with
+// 2, 4, 8, 32 workgroups per CU: 36.8, 24.4, 22.3, 23.0 / 30.9, 19.9, 17.1, 18.8 us; other mixtures agree. Entries per
+// wavefront of a tile: one-element wave groups 2, 4, 8 and whole-fiber groups 1, 2, 3, 4 at 8 workgroups per CU: 24.5,
+// 22.3, 26.3 and 27.2, 22.3, 24.9, 25.7 us (FP64).
+constexpr int kGroupWorkgroupsPerCu = 8;
+constexpr int kGroupWaveRun = 4;
+constexpr int kGroupFiberRun = 2;
+
+// One group's descriptor; returns the LDS bytes its tiles take. wave: the wave paths may be taken.
 template<typename T>
 size_t fill_group(Shape const &s, T const *const *mats, T const *const *in, T *const *out, int entries_per_tile,
                   krongroup::GroupDesc<T> &D, bool wave = false)
 {
-    D.wave = wave && kronwave::wave_shape(s.d, s.n) ? 1 : 0;
+    int const fiber_lds = krongroup::group_fiber_lds<T>(s.d, s.n);
+    D.path = !wave ? krongroup::kPass
+           : kronwave::wave_shape(s.d, s.n) ? krongroup::kWave
+           : fiber_lds > 0 ? krongroup::kWaveFiber : krongroup::kPass;
     D.d = s.d;
     D.n = s.n;
     D.stride = s.stride;
@@ -839,8 +850,13 @@ size_t fill_group(Shape const &s, T const *const *mats, T const *const *in, T *c
     D.mats = mats;
     D.in = in;
     D.out = out;
-    // a wave group's tile is cut among the workgroup's wavefronts, each with its own LDS rows
-    if (D.wave) return krongroup::kWaves * krongroup::wave_lds_elems() * sizeof(T);
+    if (D.path != krongroup::kPass)
+    {
+        // the tile is cut among the workgroup's wavefronts, each with its own LDS rows
+        int const run = D.path == krongroup::kWave ? kGroupWaveRun : kGroupFiberRun;
+        D.epw = entries_per_tile > 0 ? entries_per_tile : krongroup::kWaves * run;
+        return sizeof(T) * (D.path == krongroup::kWave ? krongroup::kWaves * krongroup::wave_lds_elems() : fiber_lds);
+    }
     return static_cast<size_t>(E) * per_entry + sizeof(void *);  // + pointer alignment
 }
 
@@ -896,9 +912,9 @@ hipError_t packed_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L,
     L.block = krongroup::kThreads;
     L.epw = table.g[0].epw;
     L.lds = lds;
-    L.resident = resident_per_cu(krongroup::kron_group_kernel<T, false>, krongroup::kThreads, lds);
+    L.resident = resident_per_cu(krongroup::kron_group_kernel<T, 1 << krongroup::kPass>, krongroup::kThreads, lds);
     if (!run || grid == 0) return hipSuccess;
-    hipLaunchKernelGGL((krongroup::kron_group_kernel<T, false>), dim3(static_cast<unsigned>(grid)), dim3(krongroup::kThreads),
+    hipLaunchKernelGGL((krongroup::kron_group_kernel<T, 1 << krongroup::kPass>), dim3(static_cast<unsigned>(grid)), dim3(krongroup::kThreads),
                        lds, stream, table);
     return hipGetLastError();
 }
@@ -1366,6 +1382,21 @@ int kronmult_adjoint_sync(int d, int n, T const *const *mats, int stride, T cons
     return static_cast<int>(hipDeviceSynchronize());
 }
 
+// AUTO: a large group that the persistent launch would sweep in passes takes a launch of its own where a faster kernel is
+// built for its shape. Measured (us, one persistent launch / with own launches): 8000 entries of d=3 n=7 FP64 20.3 /
+// 12.8; 3000 of d=5 n=4 with 6000 of d=2 n=8 28.7 / 23.0, FP32 20.9 / 14.5; 2000 of d=5 n=4 with 3000 of d=3 n=7 FP32
+// 18.5 / 17.2. Below a million elements the launch costs what it saves (500 of d=5 n=4 with 800 of d=3 n=7 each on its
+// own 10.5 against 10.8).
+constexpr long kGroupOwnLaunchElems = 1l << 20;
+
+template<typename T>
+bool group_own_launch(Shape const &s)
+{
+    if (kronwave::wave_shape(s.d, s.n) || krongroup::group_fiber_shape<T>(s.d, s.n)) return false;
+    bool const faster = reg_rho(s.d, s.n) > 0 || kronwave::wave_fiber_shape(s.d, s.n) || kronblock::block_shape<T>(s.d, s.n);
+    return faster && s.nb * s.size >= kGroupOwnLaunchElems;
+}
+
 template<typename T, typename GroupT>
 hipError_t kronmult_grouped_launch(GroupT const *groups, int count, kronmult_grouped_options_t const *options,
                                    hipStream_t stream)
@@ -1390,7 +1421,8 @@ hipError_t kronmult_grouped_launch(GroupT const *groups, int count, kronmult_gro
             return hipErrorInvalidValue;
         // groups past the first kMaxGroups always get launches of their own
         bool const pers = opt.strategy != KRONMULT_GROUPED_SEPARATE && i < krongroup::kMaxGroups &&
-                          group_persistent_ok<T>(g, s) && g.nb_batch > 0;
+                          group_persistent_ok<T>(g, s) && g.nb_batch > 0 &&
+                          !(opt.strategy == KRONMULT_GROUPED_AUTO && group_own_launch<T>(s));
         if (i < krongroup::kMaxGroups)
         {
             shapes[i] = s;
@@ -1423,7 +1455,7 @@ hipError_t kronmult_grouped_launch(GroupT const *groups, int count, kronmult_gro
     krongroup::GroupTable<T> table{};
     size_t lds = 0;
     int tiles = 0;
-    bool any_wave = false;
+    int paths = 0;
     for (int i = 0; i < count && i < krongroup::kMaxGroups; ++i)
     {
         if (!persistent[i]) continue;
@@ -1435,15 +1467,19 @@ hipError_t kronmult_grouped_launch(GroupT const *groups, int count, kronmult_gro
         table.tile_start[table.count] = tiles;
         tiles += (s.nb + D.epw - 1) / D.epw;
         if (need > lds) lds = need;
-        any_wave = any_wave || D.wave != 0;
+        paths |= 1 << D.path;
         ++table.count;
     }
     table.tile_start[table.count] = tiles;
     table.tiles = tiles;
-    int const per_cu = opt.workgroups_per_cu > 0 ? opt.workgroups_per_cu : 2;
+    int const per_cu = opt.workgroups_per_cu > 0 ? opt.workgroups_per_cu : kGroupWorkgroupsPerCu;
     long grid = static_cast<long>(device_cu_count()) * per_cu;
     if (grid > tiles) grid = tiles;
-    auto kernel = any_wave ? krongroup::kron_group_kernel<T, true> : krongroup::kron_group_kernel<T, false>;
+    constexpr int kP = 1 << krongroup::kPass, kW = 1 << krongroup::kWave, kF = 1 << krongroup::kWaveFiber;
+    auto kernel = (paths & kF) != 0 ? ((paths & kP) != 0 ? krongroup::kron_group_kernel<T, kP | kW | kF>
+                                                         : krongroup::kron_group_kernel<T, kW | kF>)
+                : (paths & kW) != 0 ? krongroup::kron_group_kernel<T, kP | kW>
+                                    : krongroup::kron_group_kernel<T, kP>;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(krongroup::kThreads), lds, stream, table);
     return hipGetLastError();
 }

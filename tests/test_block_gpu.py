@@ -95,3 +95,34 @@ def test_large_vectors_need_a_workspace(gpu, d, n, itemsize):
     db = DeviceBatch(W.random_case(380, d, n, 2, dtype=dtype), device=str(gpu), workspace="none")
     with pytest.raises(api.KronmultError):
         db.run()
+
+
+@pytest.mark.parametrize("strategy", ["auto", "persistent"])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_grouped_paths(gpu, dtype, strategy):
+    """Every path of the grouped launch, tables with and without passes, default tiles and tiles that leave wavefronts
+    without entries; a group large enough for a launch of its own under "auto" (d=5 n=4)."""
+    import torch
+    small = [(3, 5, 37), (3, 6, 90), (4, 3, 61), (4, 4, 45), (5, 3, 33), (7, 2, 18), (8, 2, 19), (2, 8, 70), (6, 2, 9)]
+    for shapes in (small, small[:2] + [(3, 7, 40), (4, 5, 21), (5, 4, 1100)]):
+        for tile in (0, 1, 6, 31):
+            bs = [W.random_case(390 + 10 * d + n, d, n, nb, stride=n + 1, distinct=nb, dtype=dtype) for d, n, nb in shapes]
+            bs = [W.HostBatch(**{**b.__dict__, "out_init": np.zeros_like(b.out_init)}) for b in bs]
+            dbs = [DeviceBatch(b, device=str(gpu)) for b in bs]
+            print(f"[grouped] {strategy} tile={tile} {shapes}", flush=True)
+            api.kronmult_batched_grouped([db.group(entries_per_tile=tile) for db in dbs], dtype=dbs[0].dtype_name,
+                                         strategy=strategy)
+            torch.cuda.synchronize()
+            for b, db in zip(bs, dbs):
+                assert np.array_equal(db.output(), oracle.kronmult(b)), (b.d, b.n, tile)
+
+
+def test_grouped_shared_outputs(gpu):
+    import torch
+    bs = [W.random_case(410 + d, d, n, nb, distinct=nb // 5) for d, n, nb in ((3, 6, 300), (5, 3, 211), (4, 4, 97))]
+    bs = bs + [grouped_by_output(b) for b in bs]
+    dbs = [DeviceBatch(b, device=str(gpu)) for b in bs]
+    api.kronmult_batched_grouped([db.group() for db in dbs], dtype="f64")
+    torch.cuda.synchronize()
+    for b, db in zip(bs, dbs):
+        assert float(np.max(np.abs(db.output() - oracle.kronmult(b)) - accumulation_bound(b, EPS[b.dtype]))) <= 0.0
