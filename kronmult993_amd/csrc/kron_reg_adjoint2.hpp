@@ -12,15 +12,22 @@
 //   * X_3 kept from the first pass (below), X_2 = A_3 X_3, dA_2, A_2^T, dA_3, A_3^T, exchange into phase 0;
 //     X_5 = x (read again) and X_4 (kept in FP32, A_5 x in FP64), dA_4, A_4^T, dA_5, A_5^T: d x in the
 //     phase-0 layout.
-// A factor gradient's per-thread partial (16 values: its 4 fibers of the mode) is reduce-scattered across
-// the wavefront in four lane-shuffle steps to one value per lane and summed over consecutive entries that
+// The entries are walked by input (kron_order.hpp). A factor gradient's per-thread partial (16 values: its 4 fibers of
+// the mode) is reduce-scattered across the wavefront in four steps (kron_lanes.hpp) to one value per lane and summed over consecutive entries that
 // share the gradient pointer; when the pointer changes, two more steps, a sum over the four wavefronts in
-// LDS and 16 atomics. d x is summed over entries that share the input gradient and leaves through one LDS
+// LDS after the next exchange's barrier and 16 atomics. d x is summed over entries that share the input gradient and leaves through one LDS
 // exchange into the coalesced phase-2 layout.
+//
+// What bounds it: two workgroups per CU (250 registers, 66 KB of LDS in FP64) hide little of the chains' latency; the
+// FMAs of a batch take 68 us. d=6 n=4, 128 x 64 pairs listed by output, FP64 / FP32: 250 / 141 us in the natural order
+// (33.5 M input-gradient atomics), 195 walked by input with the sums across lanes in the vector ALU, 189 / 112 with x
+// staged by LDS-DMA and the gradients' flush behind the exchanges' barriers; the input gradient alone 69 / 45 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include "kron_lanes.hpp"
+#include "kron_order.hpp"
 #include "kron_reg.hpp"
 
 namespace kronregadj2
@@ -81,7 +88,6 @@ __device__ __forceinline__ void partial_half(T const (&h)[kR], T const (&x)[kR],
 {
     constexpr int S = stride_of(M);
     constexpr int O = S == 4 ? 1 : 4;
-    bool const b5 = (lane >> 5) & 1;
 #pragma unroll
     for (int k = 0; k < 8; ++k)
     {
@@ -93,8 +99,7 @@ __device__ __forceinline__ void partial_half(T const (&h)[kR], T const (&x)[kR],
             lo = fma(h[r0 * S + f * O], x[c0 * S + f * O], lo);
             hi = fma(h[r1 * S + f * O], x[c1 * S + f * O], hi);
         }
-        T const mine = b5 ? hi : lo, other = b5 ? lo : hi;
-        q8[k] = mine + __shfl_xor(other, 32);
+        q8[k] = kronlanes::fold<32>(lo, hi, lane);
     }
 }
 
@@ -102,52 +107,50 @@ template<typename T>
 __device__ __forceinline__ T reduce_scatter8(T (&q8)[8], int lane)
 {
     T q4[4], q2[2];
-    bool const b4 = (lane >> 4) & 1, b3 = (lane >> 3) & 1, b2 = (lane >> 2) & 1;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-    {
-        T const mine = b4 ? q8[k + 4] : q8[k], other = b4 ? q8[k] : q8[k + 4];
-        q4[k] = mine + __shfl_xor(other, 16);
-    }
+    for (int k = 0; k < 4; ++k) q4[k] = kronlanes::fold<16>(q8[k], q8[k + 4], lane);
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
-    {
-        T const mine = b3 ? q4[k + 2] : q4[k], other = b3 ? q4[k] : q4[k + 2];
-        q2[k] = mine + __shfl_xor(other, 8);
-    }
-    T const mine = b2 ? q2[1] : q2[0], other = b2 ? q2[0] : q2[1];
-    return mine + __shfl_xor(other, 4);
+    for (int k = 0; k < 2; ++k) q2[k] = kronlanes::fold<8>(q4[k], q4[k + 2], lane);
+    return kronlanes::fold<4>(q2[0], q2[1], lane);
 }
 
-// add a run's dA partial (one value per lane, in the order above) to the gradient: lanes 0..3 of each
-// quad hold partials of one index; the four wavefronts meet in red[]
-template<typename T>
-__device__ __forceinline__ void flush_gradient(T value, T *g_generic, int stride, T *red, int t)
+// A run's dA_M partial (one value per lane, in the order above; lanes 0..3 of each quad hold partials of one index) into
+// its wavefront's row of red, index 4 r + c.
+template<typename T, int M>
+__device__ __forceinline__ void publish_gradient(T value, T *red, int t)
 {
     int const lane = t & 63, wave = t >> 6;
-    value += __shfl_xor(value, 1);
-    value += __shfl_xor(value, 2);
+    value = kronlanes::add<1>(value);
+    value = kronlanes::add<2>(value);
     int const idx = ((lane >> 5) & 1) * 8 + ((lane >> 4) & 1) * 4 + ((lane >> 3) & 1) * 2 + ((lane >> 2) & 1);
-    if ((lane & 3) == 0) red[wave * 16 + idx] = value;
-    lds_barrier();
-    if (t < 16)
+    if ((lane & 3) == 0) red[(M * kWaves + wave) * 16 + idx] = value;
+}
+
+// The published gradients of the modes in `mask`, after a barrier: 16 threads per mode add the four wavefronts' rows and
+// make one atomic each. The barrier is the one of the exchange that follows; the rows are written again only in the
+// next entry, several barriers later. (With two barriers of its own per gradient, the d=6 batch took 195 us.)
+template<typename T>
+__device__ __forceinline__ void flush_gradients(unsigned mask, T *const *gA, int stride, T const *red, int t)
+{
+    int const m = t >> 4, i = t & 15;
+    if (m < 6 && ((mask >> m) & 1u))
     {
-        T s = red[t];
+        T s = red[m * kWaves * 16 + i];
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) s += red[w * 16 + t];
-        global_ptr<T> g = as_global(g_generic);
-        atomicAdd((T *)(g + (t >> 2) + (t & 3) * stride), s);  // index 4 r + c: dA[r][c]
+        for (int w = 1; w < kWaves; ++w) s += red[(m * kWaves + w) * 16 + i];
+        global_ptr<T> g = as_global(gA[m]);
+        atomicAdd((T *)(g + (i >> 2) + (i & 3) * stride), s);  // index 4 r + c: dA[r][c]
     }
-    lds_barrier();  // red[] free for the next flush
 }
 
 // exchange the vector from the layout of phase A to that of phase B through LDS (the forward's exchange
-// swizzle on both sides)
-template<typename T, int A, int B>
-__device__ __forceinline__ void exchange(T *lds, T (&v)[kR], int t)
+// swizzle on both sides); between: what every thread does after the first barrier
+template<typename T, int A, int B, typename F = kronreg::NoHook>
+__device__ __forceinline__ void exchange(T *lds, T (&v)[kR], int t, F const &between = F())
 {
     using SW = kronplan::PlanSwizzle<PL, T, 1>;
     lds_barrier();
+    between();
 #pragma unroll
     for (int j = 0; j < kR; ++j) lds[SW::phys(PL::elem(A, t, j))] = v[j];
     lds_barrier();
@@ -188,6 +191,33 @@ __device__ __forceinline__ void restore(T const *buf, T (&v)[kR], int t)
     for (int j = 0; j < kR; ++j) v[j] = buf[j * kP + t];
 }
 
+// FP64: x goes through LDS, by LDS-DMA in the swizzled order of the forward sweep's staging (kron_reg.hpp), into the
+// buffer that X_3 has left; there it serves X_5 and, when the next entry has the same input (the walk by input), the
+// next X chain. Read straight from memory in the phase-0 layout, 16 consecutive values per thread, every load
+// instruction touches 64 lines, twice per entry.
+template<typename T>
+constexpr bool stage_x_ok()
+{
+    return sizeof(T) == 8 && kronreg::Lds<T, PL>::dma_ok();
+}
+
+template<typename T>
+__device__ __forceinline__ void stage_x(T *buf, T const *src, int t)
+{
+    if ((reinterpret_cast<uintptr_t>(src) & 15) == 0)
+        kronreg::Lds<T, PL>::dma_input(buf, src, t);
+    else
+    {
+        T tmp[kR];
+        kronreg::load_input<T, PL>(src, tmp, t);
+        kronreg::Lds<T, PL>::store_input(buf, tmp, t);
+    }
+}
+__device__ __forceinline__ void stage_wait()
+{
+    __builtin_amdgcn_s_waitcnt(kronreg::kWaitVmcnt0);  // this wavefront's LDS-DMA loads have landed
+}
+
 template<typename T>
 __global__ void __launch_bounds__(kP)
     kron_reg_adjoint2_kernel(int nb, int epw, T const *const *__restrict__ mats, int stride,
@@ -196,17 +226,19 @@ __global__ void __launch_bounds__(kP)
 {
     static_assert(PL::NPHASE == 3 && PL::elem(2, 1, 0) == 1 && PL::elem(2, 0, 1) == kP,
                   "phase 2 is element j * P + t");
-    constexpr bool kKeep = true;
     constexpr bool kKeep4 = keep_x4<T>();
-    __shared__ __attribute__((aligned(16))) T lds[PL::SIZE * (1 + (kKeep ? 1 : 0) + (kKeep4 ? 1 : 0))];
-    __shared__ T red[kWaves * 16];
+    constexpr bool kStageX = stage_x_ok<T>();
+    using L = kronreg::Lds<T, PL>;
+    __shared__ __attribute__((aligned(16))) T lds[PL::SIZE * (2 + (kKeep4 ? 1 : 0))];
+    __shared__ T red[6 * kWaves * 16];
+    __shared__ int first_shared;
     T *const x3buf = lds + PL::SIZE;
     T *const x4buf = lds + 2 * PL::SIZE;
     int const t = threadIdx.x;
     int const lane = t & 63;
-    int const e0 = kronreg::xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
-    if (e0 >= e1) return;
+    kronorder::Walk walk = kronorder::walk(gin, nb, epw, &first_shared);
+    int e = walk.next();
+    if (e < 0) return;
     bool const want_mats = gmats != nullptr;
     bool const want_input = gin != nullptr;
 
@@ -226,43 +258,68 @@ __global__ void __launch_bounds__(kP)
 #pragma unroll
         for (int j = 0; j < kR; ++j) dst[j] = g[j * kP + t];
     };
-    if constexpr (kPreG) load_g(e0, gpre);
+    if constexpr (kPreG) load_g(e, gpre);
 
-    for (int e = e0; e < e1; ++e)
+    unsigned pending = 0;  // modes whose gradients (of entry pending_from) are published and not yet added
+    int pending_from = 0;
+    T const *staged = nullptr;  // the input held in the X_3 buffer (kStageX)
+    int en = -1;  // the entry after e
+    for (; e >= 0; e = en)
     {
-        bool const last = e + 1 >= e1;
+        en = walk.next();
+        bool const last = en < 0;
         T const *const *A = mats + static_cast<size_t>(e) * 6;
         T h[kR], v[kR], xs[kR];
-        // one dA step: partial of mode M from (h, x), run sum, flush when the next entry's pointer differs
+        // one dA step: partial of mode M from (h, x), run sum, published when the next entry's pointer differs
         auto grad = [&](auto mc, T const (&x)[kR]) {
             constexpr int M = decltype(mc)::value;
             T q8[8];
             partial_half<T, M>(h, x, q8, lane);
             gacc[M] += reduce_scatter8(q8, lane);
             T *const gA = gmats[static_cast<size_t>(e) * 6 + M];
-            if (last || gmats[static_cast<size_t>(e + 1) * 6 + M] != gA)
+            if (last || gmats[static_cast<size_t>(en) * 6 + M] != gA)
             {
-                flush_gradient(gacc[M], gA, stride, red, t);
+                publish_gradient<T, M>(gacc[M], red, t);
                 gacc[M] = T(0);
+                pending |= 1u << M;
+                pending_from = e;
             }
+        };
+        auto flush = [&]() {
+            if (pending != 0)
+                flush_gradients(pending, gmats + static_cast<size_t>(pending_from) * 6, stride, red, t);
+            pending = 0;
         };
         // cotangent in the phase-2 layout: element j * 256 + t
         if constexpr (kPreG)
         {
 #pragma unroll
             for (int j = 0; j < kR; ++j) h[j] = gpre[j];
-            if (!last) load_g(e + 1, gpre);
+            if (!last) load_g(en, gpre);
         }
         else
             load_g(e, h);
         if (want_mats)
         {
-            load_x(in[e], v, t);
+            if constexpr (kStageX)
+            {
+                if (staged != in[e])
+                {
+                    lds_barrier();  // every thread is done with the buffer
+                    stage_x(x3buf, in[e], t);
+                    staged = in[e];
+                    stage_wait();
+                    lds_barrier();
+                }
+                L::read0_dma(x3buf, v, t);
+            }
+            else
+                load_x(in[e], v, t);
             contract<T, 5, false>(v, A[5], stride);
             if constexpr (kKeep4) keep(x4buf, v, t);  // X_4
             contract<T, 4, false>(v, A[4], stride);
-            exchange<T, 0, 1>(lds, v, t);
-            if constexpr (kKeep) keep(x3buf, v, t);   // X_3
+            exchange<T, 0, 1>(lds, v, t, flush);  // (the previous entry's dA_4, dA_5)
+            keep(x3buf, v, t);   // X_3
             contract<T, 3, false>(v, A[3], stride);
             contract<T, 2, false>(v, A[2], stride);
             exchange<T, 1, 2>(lds, v, t);
@@ -274,18 +331,10 @@ __global__ void __launch_bounds__(kP)
         contract<T, 0, true>(h, A[0], stride);  // H_1
         if (want_mats) grad(std::integral_constant<int, 1>(), xs);
         contract<T, 1, true>(h, A[1], stride);  // H_2
-        exchange<T, 2, 1>(lds, h, t);
+        exchange<T, 2, 1>(lds, h, t, flush);  // dA_0, dA_1
         if (want_mats)
         {
-            if constexpr (kKeep)
-                restore(x3buf, v, t);
-            else
-            {
-                load_x(in[e], v, t);
-                contract<T, 5, false>(v, A[5], stride);
-                contract<T, 4, false>(v, A[4], stride);
-                exchange<T, 0, 1>(lds, v, t);
-            }
+            restore(x3buf, v, t);
 #pragma unroll
             for (int j = 0; j < kR; ++j) xs[j] = v[j];  // X_3
             contract<T, 3, false>(v, A[3], stride);      // X_2
@@ -294,10 +343,22 @@ __global__ void __launch_bounds__(kP)
         contract<T, 2, true>(h, A[2], stride);  // H_3
         if (want_mats) grad(std::integral_constant<int, 3>(), xs);
         contract<T, 3, true>(h, A[3], stride);  // H_4
-        exchange<T, 1, 0>(lds, h, t);
+        exchange<T, 1, 0>(lds, h, t, [&]() {
+            flush();  // dA_2, dA_3
+            // every thread has read X_3: x into its buffer, for X_5 and for the next entry if it has the same input
+            if constexpr (kStageX)
+                if (want_mats) stage_x(x3buf, in[e], t);
+        });
         if (want_mats)
         {
-            load_x(in[e], xs, t);  // X_5
+            if constexpr (kStageX)
+            {
+                stage_wait();
+                lds_barrier();
+                L::read0_dma(x3buf, xs, t);  // X_5
+            }
+            else
+                load_x(in[e], xs, t);
             if constexpr (kKeep4)
                 restore(x4buf, v, t);
             else
@@ -315,7 +376,7 @@ __global__ void __launch_bounds__(kP)
             contract<T, 5, true>(h, A[5], stride);  // d x, phase-0 layout
 #pragma unroll
             for (int j = 0; j < kR; ++j) dxacc[j] += h[j];
-            if (last || gin[e + 1] != gin[e])
+            if (last || gin[en] != gin[e])
             {
                 exchange<T, 0, 2>(lds, dxacc, t);
                 global_ptr<T> gi = as_global(gin[e]);
@@ -327,6 +388,11 @@ __global__ void __launch_bounds__(kP)
                 }
             }
         }
+    }
+    if (pending != 0)
+    {
+        lds_barrier();
+        flush_gradients(pending, gmats + static_cast<size_t>(pending_from) * 6, stride, red, t);
     }
 }
 
