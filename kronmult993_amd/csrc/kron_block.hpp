@@ -45,9 +45,9 @@ struct Block
     static constexpr int NFIB = S / N;
     static constexpr int F = (NFIB + P - 1) / P;  // fibers per thread
     static constexpr int GR = 16 / static_cast<int>(sizeof(T));
-    // LDS: canonical order; for n = 8 every row of 8 is followed by 16 bytes, so that the fastest mode's fibers,
-    // a row apart across lanes, start in different banks (other n: the row length does that by itself)
-    static constexpr int PAD = N == 8 ? GR : 0;
+    // LDS: canonical order; for n = 8, and n = 4 in FP64, every row of n is followed by 16 bytes, so that the fastest
+    // mode's fibers, a row apart across lanes, start in different banks (other n: the row length does that by itself)
+    static constexpr int PAD = N == 8 || (N == 4 && sizeof(T) == 8) ? GR : 0;
     static constexpr int LDS = S + PAD * (S / N);
     static constexpr int NGRAN = S / GR, REM = S % GR;
     static constexpr int CPT = (NGRAN + P - 1) / P;
@@ -72,6 +72,13 @@ struct Block
         for (int c = 0; c < CPT; ++c)
             if (granule(c, t)) pre[c] = *(kronreg::global_ptr<VU const>)(src + (c * P + t) * GR);
         if (REM > 0 && t < REM) pre_rem = src[NGRAN * GR + t];
+    }
+    // the values of load are in the registers
+    __device__ __forceinline__ void arrived()
+    {
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) asm volatile("" : "+v"(pre[c]));
+        if (REM > 0) asm volatile("" : "+v"(pre_rem));
     }
     __device__ __forceinline__ void store(T *lds, int t) const
     {

@@ -21,29 +21,47 @@ constexpr int kScan = 4096;  // pointers looked at (16 loads per thread of a 256
 
 struct Walk
 {
-    int nb, period, rows;  // entry of step v: v / rows + (v % rows) * period
-    int v, end;            // this workgroup's next step and the end of its steps
+    int nb, period, rows;  // the entry of column c, row r is c + r * period
+    int c, r, left;        // this workgroup's next step and the number of its steps
 
     // the next entry, or -1 (a step past the batch, in the last row, is left out)
     __device__ __forceinline__ int next()
     {
-        while (v < end)
+        while (left > 0)
         {
-            int const c = v / rows;
-            int const k = c + (v - c * rows) * period;
-            ++v;
+            int const k = c + r * period;
+            --left;
+            if (++r == rows)
+            {
+                r = 0;
+                ++c;
+            }
             if (k < nb) return k;
         }
         return -1;
     }
 };
 
-// `run` entries per workgroup in the natural order; ptr may be null (natural order). Every thread calls it.
+// Whether a factor gradient of entry 0 is one of the entries a third and two thirds into the batch too (every wavefront
+// finds the same answer; d <= 64).
 template<typename T>
-__device__ __forceinline__ Walk walk(T *const *ptr, int nb, int run, int *shared_min)
+__device__ __forceinline__ bool shared_gradients(T *const *gmats, int nb, int d)
+{
+    if (gmats == nullptr) return false;
+    int const lane = static_cast<int>(threadIdx.x) & 63, m = lane < d ? lane : 0;
+    T *const first = kronreg::as_global(gmats)[m];
+    bool const same = first == kronreg::as_global(gmats)[static_cast<size_t>(nb / 3) * d + m] ||
+                      first == kronreg::as_global(gmats)[static_cast<size_t>(nb - 1 - nb / 3) * d + m];
+    return __ballot(same) != 0;
+}
+
+// This workgroup's part of the batch, cut into `groups` (a multiple of 8, at most the grid) equal parts; the workgroups
+// past them get none. ptr may be null (natural order). Every thread calls it.
+template<typename T>
+__device__ __forceinline__ Walk walk(T *const *ptr, int nb, int groups, int *shared_min)
 {
     int period = 1;
-    if (ptr != nullptr && run > 1)
+    if (ptr != nullptr && nb > groups)
     {
         if (threadIdx.x == 0) *shared_min = INT_MAX;
         __syncthreads();
@@ -62,22 +80,19 @@ __device__ __forceinline__ Walk walk(T *const *ptr, int nb, int run, int *shared
     Walk w;
     w.nb = nb;
     w.period = period;
-    w.rows = (nb + period - 1) / period;
-    int const index = kronreg::xcd_run_index();
-    int per = run;
-    if (period > 1)
-    {
-        // steps, those past the batch among them, in equal parts
-        long const steps = static_cast<long>(w.rows) * period;
-        per = static_cast<int>((steps + gridDim.x - 1) / gridDim.x);
-        long const v0 = static_cast<long>(index) * per;
-        w.v = static_cast<int>(v0 < steps ? v0 : steps);
-        w.end = static_cast<int>(v0 + per < steps ? v0 + per : steps);
-        return w;
-    }
-    w.rows = nb;  // one column
-    w.v = nb - 1 < static_cast<long>(index) * per ? nb : index * per;
-    w.end = nb - w.v > per ? w.v + per : nb;
+    w.rows = static_cast<int>((static_cast<long>(nb) + period - 1) / period);
+    // consecutive parts on one XCD (kronreg::xcd_run_index, over `groups`)
+    int const per_xcd = groups >> 3, slot = static_cast<int>(blockIdx.x >> 3);
+    long const index = static_cast<long>(blockIdx.x & 7) * per_xcd + slot;
+    // the steps, those past the batch among them, in parts that differ by one at most
+    long const steps = static_cast<long>(w.rows) * period;
+    long const v0 = slot < per_xcd ? index * steps / groups : steps;
+    long const v1 = slot < per_xcd ? (index + 1) * steps / groups : steps;
+    // (in scalar registers: the divisions leave them in vector registers)
+    w.left = __builtin_amdgcn_readfirstlane(static_cast<int>(v1 - v0));
+    w.c = __builtin_amdgcn_readfirstlane(static_cast<int>(v0 / w.rows));
+    w.r = __builtin_amdgcn_readfirstlane(static_cast<int>(v0 - v0 / w.rows * w.rows));
+    w.rows = __builtin_amdgcn_readfirstlane(w.rows);
     return w;
 }
 

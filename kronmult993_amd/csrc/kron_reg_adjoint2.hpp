@@ -220,7 +220,7 @@ __device__ __forceinline__ void stage_wait()
 
 template<typename T>
 __global__ void __launch_bounds__(kP)
-    kron_reg_adjoint2_kernel(int nb, int epw, T const *const *__restrict__ mats, int stride,
+    kron_reg_adjoint2_kernel(int nb, T const *const *__restrict__ mats, int stride,
                              T const *const *__restrict__ in, T const *const *__restrict__ gout,
                              T *const *__restrict__ gin, T *const *__restrict__ gmats)
 {
@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(kP)
     T *const x4buf = lds + 2 * PL::SIZE;
     int const t = threadIdx.x;
     int const lane = t & 63;
-    kronorder::Walk walk = kronorder::walk(gin, nb, epw, &first_shared);
+    kronorder::Walk walk = kronorder::walk(gin, nb, static_cast<int>(gridDim.x), &first_shared);
     int e = walk.next();
     if (e < 0) return;
     bool const want_mats = gmats != nullptr;

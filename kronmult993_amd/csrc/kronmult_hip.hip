@@ -32,6 +32,7 @@
 
 #include "kron_adjoint.hpp"
 #include "kron_block.hpp"
+#include "kron_block_adjoint.hpp"
 #include "kron_final.hpp"
 #include "kron_group.hpp"
 #include "kron_mfma.hpp"
@@ -1275,14 +1276,42 @@ hipError_t adjoint2_launch(Shape const &s, T const *const *mats, T const *const 
 {
     auto kernel = kronregadj2::kron_reg_adjoint2_kernel<T>;
     int const per_cu = resident_per_cu(kernel, kronregadj2::kP, 0);
-    long const slots = static_cast<long>(device_cu_count()) * per_cu;
-    int epw = static_cast<int>((s.nb + slots - 1) / slots);
-    if (epw < 1) epw = 1;
-    long const runs = (s.nb + epw - 1) / epw;
-    long const grid = (runs + 7) / 8 * 8;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kronregadj2::kP), 0, stream, s.nb, epw, mats,
+    long const grid = (std::min<long>(s.nb, static_cast<long>(device_cu_count()) * per_cu) + 7) / 8 * 8;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kronregadj2::kP), 0, stream, s.nb, mats, s.stride, in,
+                       gout, gin, gmats);
+    return hipGetLastError();
+}
+
+// Whole entries on the block layout (kron_block_adjoint.hpp), AUTO: every resident workgroup takes an equal part of the
+// entries; where the entries share factor gradients (looked for on the device) only this many per CU do, whose longer
+// runs make fewer atomic adds to the same few addresses. Measured, 128 x 64 element pairs FP32, at 2 / 4 / 8 / all: d=4 n=5
+// 71 / 61 / 75 / 76 us, d=6 n=2 50 / 42 / 48 / 69, d=3 n=7 85 / 71 / 82 / 83.
+constexpr long kBlockAdjointSharedPerCu = 4;
+
+template<typename T, int D, int N>
+hipError_t block_adjoint_launch_dn(Shape const &s, T const *const *mats, T const *const *in, T const *const *gout,
+                                   T *const *gin, T *const *gmats, hipStream_t stream)
+{
+    constexpr int P = kronblock::block_threads<N, D>();
+    auto kernel = kronblockadj::kron_block_adjoint_kernel<T, N, D, P>;
+    long const cus = device_cu_count();
+    long const grid = (std::min<long>(s.nb, cus * resident_per_cu(kernel, P, 0)) + 7) / 8 * 8;
+    long const shared = (cus * kBlockAdjointSharedPerCu + 7) / 8 * 8;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(P), 0, stream, s.nb, static_cast<int>(shared), mats,
                        s.stride, in, gout, gin, gmats);
     return hipGetLastError();
+}
+
+template<typename T>
+hipError_t block_adjoint_launch(Shape const &s, T const *const *mats, T const *const *in, T const *const *gout,
+                                T *const *gin, T *const *gmats, hipStream_t stream)
+{
+#define KRON_BLOCK_ADJOINT_LAUNCH(D, N)                   \
+    if constexpr (kronblockadj::adjoint_shape<T>(D, N)) \
+        if (s.d == D && s.n == N) return block_adjoint_launch_dn<T, D, N>(s, mats, in, gout, gin, gmats, stream);
+    KRON_BLOCK_ADJOINT_SHAPES(KRON_BLOCK_ADJOINT_LAUNCH)
+#undef KRON_BLOCK_ADJOINT_LAUNCH
+    return hipErrorInvalidValue;
 }
 
 template<typename T>
@@ -1292,12 +1321,11 @@ hipError_t reg_adjoint_dispatch(Shape const &s, int intermediates, T const *cons
     if (s.d == 6 && s.n == 4 && intermediates == KRONMULT_ADJOINT_AUTO)
         return adjoint2_launch<T>(s, mats, in, gout, gin, gmats, stream);
     // STORE: the chain in LDS where it fits comfortably (d=3 n=8, d=4 n=4), else in registers.
-    // AUTO, measured per shape: d=4 n=8 and d=5/6 n=4 keep the chain in registers (d=6 n=4 FP64 0.58 ms
-    // against 0.78 ms recomputing, FP32 0.38 against 0.49; d=4 n=8 FP64 1.01 against 1.15 ms); d=3 n=8
-    // recomputes (FP64 three waves per SIMD: 41.7 us against 46.4 us keeping the chain; FP32 24.6 us
-    // against 24.9 us with the chain in LDS); d=4 n=4 recomputes in FP64, keeps the chain in LDS in FP32
+    // AUTO, measured per shape: d=4 n=8 FP64 keeps the chain in registers (1.01 against 1.15 ms recomputing); d=3
+    // n=8 recomputes (FP64 three waves per SIMD: 41.7 us against 46.4 us keeping the chain; FP32 24.6 us against
+    // 24.9 us with the chain in LDS); d=4 n=4 recomputes in FP64, keeps the chain in LDS in FP32
     bool const lds_ok = reg_adjoint_store_ok<T>(s);
-    bool const keep_preferred = (s.d == 4 && s.n == 8) || (s.d == 5 && s.n == 4) || (s.d == 6 && s.n == 4);
+    bool const keep_preferred = s.d == 4 && s.n == 8;
     RegAdjMode mode;
     if (intermediates == KRONMULT_ADJOINT_RECOMPUTE)
         mode = RegAdjMode::Recompute;
@@ -1356,6 +1384,8 @@ hipError_t kronmult_adjoint_launch(int d, int n, T const *const *mats, int strid
     if (err != hipSuccess) return err;
     if (nb == 0 || (gin == nullptr && gmats == nullptr)) return hipSuccess;
     if (mats == nullptr || gout == nullptr || (gmats != nullptr && in == nullptr)) return hipErrorInvalidValue;
+    if (intermediates == KRONMULT_ADJOINT_AUTO && kronblockadj::adjoint_shape<T>(s.d, s.n))
+        return block_adjoint_launch<T>(s, mats, in, gout, gin, gmats, stream);
     if (reg_adjoint_ok<T>(s, intermediates))
         return reg_adjoint_dispatch<T>(s, intermediates, mats, in, gout, gin, gmats, stream);
     if (p.ws_elems > 0 && ws == nullptr) return hipErrorInvalidValue;

@@ -46,3 +46,20 @@ def test_two_modes_per_phase_walks(gpu, nb, inputs, gap, dtype):
 def test_inputs_without_a_period(gpu):
     rng = np.random.default_rng(7)
     _check(_batch(510, 6, 4, 1200, rng.integers(0, 37, 1200), 5, 16, np.float64), gpu)
+
+
+BLOCK_SHAPES = [(3, 5), (3, 6), (3, 7), (4, 3), (4, 5), (4, 6), (4, 7), (4, 8), (5, 3), (5, 4), (5, 5), (6, 2), (6, 3)]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("d,n", BLOCK_SHAPES)
+def test_block_adjoint(gpu, d, n, dtype):
+    """Few entries; a batch listed by output with runs of several entries per workgroup and a last row that is not full
+    (shared factors: the smaller grid); inputs of their own with factors that take turns; one gradient only."""
+    _check(_batch(520 + 9 * d + n, d, n, 5, 5, 2, 2, dtype, 1), gpu)
+    nb = 2600 if n ** d <= 700 else 1100
+    _check(_batch(530 + 9 * d + n, d, n, nb - 3, 13, 1, 13, dtype, n % 2), gpu)
+    _check(_batch(540 + 9 * d + n, d, n, nb + 1, nb + 1, 19, 4, dtype), gpu)
+    b = _batch(550 + 9 * d + n, d, n, 90, 7, 5, 6, dtype)
+    _check(b, gpu, want_mats=False)
+    _check(b, gpu, want_input=False)
