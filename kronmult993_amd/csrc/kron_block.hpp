@@ -389,8 +389,9 @@ constexpr int pass_threads()
 }
 
 // Blocks per workgroup: one where several workgroups share a CU and hide each other's start (up to 256 threads), else
-// about 8 workgroups per CU, which read ahead (n=8 FP64: 4.6 TB/s against 3.6 with one block per workgroup).
+// workgroups of 128 wavefronts in total per CU, which read ahead (n=8 FP64: 16 workgroups per CU 4.7 TB/s, 8 4.5, with
+// one block per workgroup 3.6; n=10 FP64 25 entries: 8 per CU 194 us, 16 210).
 constexpr int kPassOneBlockThreads = 256;
-constexpr int kPassWorkgroupsPerCu = 8;
+constexpr int kPassWavesPerCu = 128;
 
 } // namespace kronblock

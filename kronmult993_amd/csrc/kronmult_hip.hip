@@ -738,13 +738,20 @@ hipError_t block_passes_dn(Shape const &s, Launch &L, T const *const *mats, T co
     long const items = static_cast<long>(s.nb) * kPerEntry;
     long block_run = 1;
     if (P > kronblock::kPassOneBlockThreads)
-        block_run = std::max(1l, (items + cus * kronblock::kPassWorkgroupsPerCu - 1) / (cus * kronblock::kPassWorkgroupsPerCu));
+    {
+        long const slots = cus * (kronblock::kPassWavesPerCu * 64 / P);
+        block_run = std::max(1l, (items + slots - 1) / slots);
+    }
     long const block_grid = ((items + block_run - 1) / block_run + 7) / 8 * 8;
     // entries per wavefront of the second pass
     long const waves = static_cast<long>(kTiles) * (N / RB) * s.nb;
     long const final_run = std::min<long>(kronfinal::kMaxRun, std::max(1l, waves / (cus * kronfinal::kWavesPerCu)));
-    long const groups = (s.nb + final_run * kronfinal::kWaves - 1) / (final_run * kronfinal::kWaves);
-    long const final_grid = (groups * kTiles * (N / RB) + 7) / 8 * 8;
+    bool const is_long = final_run >= kronfinal::kLongRun;
+    long const per_group = final_run * (is_long ? kronfinal::parts<N, RB, true>() : kronfinal::parts<N, RB, false>());
+    long const groups = (s.nb + per_group - 1) / per_group;
+    int const row_groups =
+        N / RB / (is_long ? kronfinal::shared_rows<N, RB, true>() : kronfinal::shared_rows<N, RB, false>());
+    long const final_grid = (groups * kTiles * row_groups + 7) / 8 * 8;
     L.family = KRONMULT_FAMILY_FIBER;
     L.block = P;
     L.epw = 1;
@@ -753,7 +760,7 @@ hipError_t block_passes_dn(Shape const &s, Launch &L, T const *const *mats, T co
     L.workspace = true;
     if (items > INT_MAX - 8 || final_grid > INT_MAX) return hipErrorInvalidValue;
     auto pass = kronblock::kron_block_pass_kernel<T, N, G, Q, P>;
-    auto last = kronfinal::kron_final_kernel<T, N, RB>;
+    auto last = is_long ? kronfinal::kron_final_kernel<T, N, RB, true> : kronfinal::kron_final_kernel<T, N, RB, false>;
     if (!run) L.resident = resident_per_cu(pass, P, 0);
     if (!run) return hipSuccess;
     hipLaunchKernelGGL(pass, dim3(static_cast<unsigned>(block_grid)), dim3(P), 0, stream, static_cast<int>(items),

@@ -88,6 +88,15 @@ def test_large_vectors_run_lengths(gpu):
     _check(W.random_case(372, 5, 9, 300, shared_factors=40, distinct=5, dtype=np.float64), gpu)
 
 
+@pytest.mark.parametrize("d,n,dtype,nb", [(5, 8, np.float64, 1026), (5, 8, np.float32, 1030), (5, 10, np.float32, 515),
+                                          (5, 7, np.float64, 1029), (5, 10, np.float64, 513)])
+def test_large_vectors_long_runs(gpu, d, n, dtype, nb):
+    """Runs of four entries and more: row blocks that share a workgroup, reads past the caches; a last workgroup with
+    a short part or without its second one."""
+    _check(shift_odd_inputs(W.random_case(390 + n, d, n, nb, stride=n + n % 3, shared_factors=41, distinct=5,
+                                          dtype=dtype)), gpu)
+
+
 @pytest.mark.parametrize("d,n,itemsize", [(4, 10, 8), (5, 7, 8), (6, 5, 8), (6, 10, 4)])
 def test_large_vectors_need_a_workspace(gpu, d, n, itemsize):
     dtype = np.float64 if itemsize == 8 else np.float32
