@@ -20,6 +20,7 @@
 
 #include <cstdint>
 #include <type_traits>
+#include <type_traits>
 
 #include "kron_plan.hpp"
 
@@ -132,9 +133,8 @@ constexpr bool coef_in_lds()
     return PL::kN >= 8;
 }
 
-// The forward sweep's choice: FP32 factors of n = 8 (64 values) still fit in scalar registers, and scalar
-// loads measured faster there (d=3 n=8: 9.8 against 10.7 us; d=4 n=8: 190 against 196 us); FP64 ones
-// (128 registers) are staged in LDS (scalar: 22.2 against 17.9 us, 320 against 299 us).
+// The forward sweep's choice: FP64 factors of n = 8 (128 registers) are staged in LDS (scalar: 22.2 against 17.9 us,
+// 320 against 299 us); FP32 ones are kept in the lanes (LaneFactors below).
 template<typename T, typename PL>
 constexpr bool fwd_coef_in_lds()
 {
@@ -178,14 +178,106 @@ struct Coef
     }
 };
 
+// FP32 factors stay in the lanes and the products run on the matrix cores, V_MFMA_F32_4X4X1_16B_F32: sixteen blocks
+// of four lanes, where lane 4b + i supplies row i of the left operand, lane 4b + j column j of the right one and
+// receives its column's four results. With one block of the left operand broadcast to all sixteen (CBSZ = 4, ABID =
+// its number) every lane keeps its own fiber: y[r] += A[r][k] x[k] for four rows r in one instruction, which is the
+// fused step of the other kernels, k by k from zero -- its result is bit-identical (measured, subnormals, infinities
+// and NaN included). A register of 64 lanes holds sixteen blocks of four rows of one column: four factors of n = 4 or
+// one of n = 8, so an entry's factors are two loads per lane at most, and no scalar registers.
+// Rate, measured: 135 TFLOP/s against 78 for v_fma_f32. Against FMA chains with scalar factor loads: d=4 n=4 30000
+// entries 29.6 -> 16.2 us, d=5 n=4 16000 entries 30.3 -> 26.0, d=6 n=4 8192 entries 46.5 -> 41.9 (three terms 85.1 ->
+// 71.0), d=3 n=8 8192 entries 9.5 -> 7.7, d=4 n=8 8192 entries 56.8 -> 45.6; a few hundred entries 0 to 10% less.
+template<typename T, typename PL>
+constexpr bool lane_factors()
+{
+    return sizeof(T) == 4;
+}
+
+typedef float Quad __attribute__((ext_vector_type(4)));
+
+template<int I, int E, typename F>
+__device__ __forceinline__ void static_for(F const &f)
+{
+    if constexpr (I < E)
+    {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, E>(f);
+    }
+}
+
+template<typename PL>
+struct LaneFactors
+{
+    static constexpr int N = PL::kN, H = N / 4;
+    static_assert(N % 4 == 0, "whole blocks of four rows");
+    static constexpr int kBlocks = PL::kD * H * N;  // block (m * H + h) * N + k: rows 4h .. 4h+3 of column k of factor m
+    static constexpr int V = (kBlocks + 15) / 16;
+    float a[V];
+
+    static __device__ __forceinline__ int block(int i, int lane)
+    {
+        int const q = i * 16 + (lane >> 2);
+        return q < kBlocks ? q : kBlocks - 1;
+    }
+    // The factors' addresses are read one step before their values, so that no load waits for another one.
+    struct Next
+    {
+        float const *ptr[V];
+        __device__ __forceinline__ void address(float const *const *A_list, int lane)
+        {
+#pragma unroll
+            for (int i = 0; i < V; ++i) ptr[i] = A_list[block(i, lane) / (H * N)];
+        }
+        __device__ __forceinline__ void load(float (&a)[V], int stride, int lane) const
+        {
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+            {
+                int const q = block(i, lane);
+                a[i] = as_global(ptr[i])[4 * (q / N % H) + (lane & 3) + (q % N) * stride];
+            }
+        }
+    };
+
+    // contract mode M, which has stride S in the register index
+    template<int M, int R, int S>
+    __device__ __forceinline__ void contract(float (&v)[R]) const
+    {
+        constexpr int F = R / N;  // fibers of this lane
+        Quad y[F][H];
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+#pragma unroll
+            for (int h = 0; h < H; ++h) y[f][h] = Quad{0.f, 0.f, 0.f, 0.f};
+        static_for<0, N * H>([&](auto step) {
+            constexpr int k = step.value / H, h = step.value % H, q = (M * H + h) * N + k;
+#pragma unroll
+            for (int f = 0; f < F; ++f)
+                y[f][h] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[q / 16], v[f / S * S * N + f % S + k * S], y[f][h], 4,
+                                                             q % 16, 0);
+        });
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+#pragma unroll
+            for (int r = 0; r < N; ++r) v[f / S * S * N + f % S + r * S] = y[f][r / 4][r % 4];
+    }
+};
+
+// What the phases take the factors from: the lanes, an LDS copy, or (FP64 n = 4) nothing but the pointers.
+template<typename T, typename PL>
+using PhaseFactors = std::conditional_t<lane_factors<T, PL>(), LaneFactors<PL>, T const *>;
+
 // contract modes M, M-1, ..., LO of phase PH (fastest first)
 template<typename T, typename PL, int PH, int M>
 __device__ __forceinline__ void contract_phase(T (&v)[PL::R], T const *const *__restrict__ A_list, int stride,
-                                               T const *coef)
+                                               PhaseFactors<T, PL> const &coef)
 {
     if constexpr (M >= PL::lo(PH))
     {
-        if constexpr (fwd_coef_in_lds<T, PL>())
+        if constexpr (lane_factors<T, PL>())
+            coef.template contract<M, PL::R, PL::reg_stride(M - PL::lo(PH))>(v);
+        else if constexpr (fwd_coef_in_lds<T, PL>())
             contract_mode_lds<T, PL::kN, PL::R, PL::reg_stride(M - PL::lo(PH))>(v, coef + M * PL::kN * PL::kN);
         else
             contract_mode<T, PL::kN, PL::R, PL::reg_stride(M - PL::lo(PH))>(v, A_list[M], stride);
@@ -453,7 +545,7 @@ constexpr bool raise_priority_in_contraction()
 // contraction), when the LDS tensor is no longer needed by this thread
 template<typename T, typename PL, int PH, bool PRIO = false, typename F = NoHook>
 __device__ __forceinline__ void run_phases(T *lds, T (&v)[PL::R], T const *const *__restrict__ A_list, int stride,
-                                           T const *coef, int t, F const &after_last_read = F())
+                                           PhaseFactors<T, PL> const &coef, int t, F const &after_last_read = F())
 {
     if constexpr (PH + 1 == PL::NPHASE) after_last_read();
     if constexpr (raise_priority_in_contraction<T, PL, PRIO>()) __builtin_amdgcn_s_setprio(1);
@@ -537,11 +629,12 @@ constexpr bool dma_staging()
 // Waves per SIMD the register allocator must allow (the kernel's VGPR budget is 512 / waves): chosen so
 // that an extra workgroup fits per CU where the plan is a few registers over a threshold. The DMA-staged
 // d=6 n=4 FP64 sweep fits 128 registers once the prefetch registers are gone (4 workgroups per CU: 49.5
-// against 53.3 us at 3 and 55.6 us with register staging); three was the best without DMA (168 registers).
+// against 53.3 us at 3 and 55.6 us with register staging); three was the best without DMA (168 registers). The FP32
+// n = 4 plans fit 128 as well, so as many workgroups are resident as with factors in scalar registers.
 template<typename T, typename PL>
 constexpr int min_waves_per_simd()
 {
-    return dma_staging<T, PL>() ? 4 : 1;
+    return dma_staging<T, PL>() || (lane_factors<T, PL>() && PL::kN == 4) ? 4 : 1;
 }
 
 // ORDERED: the accumulator is flushed per piece (flush_piece) instead of with atomics; ws is read only then.
@@ -629,37 +722,72 @@ __global__ void __launch_bounds__(PL::P) __attribute__((amdgpu_waves_per_eu(min_
     };
     T pre[PL::R];
     T pre_coef[kCoefLds ? Coef<T, PL>::kPerThread : 1];
-    load_input<T, PL>(in[e0], pre, t);
-    if constexpr (kCoefLds) Coef<T, PL>::load(mats + static_cast<size_t>(e0) * PL::kD, stride, pre_coef, t);
-
-    for (int e = e0; e < e1; ++e)
+    if constexpr (lane_factors<T, PL>())
     {
-        // With factors staged in LDS the previous run is flushed before the sweep, not after it: with the
-        // branch between the last phase and the accumulation, the compiler issued that phase's coefficient
-        // reads (64 values for n = 8 FP64) above the branch and its FMAs below, holding all of them live
-        // (220 VGPRs; 120 flushing first; d=4 n=8: 236 -> 210 us per launch). The other plans flush after
-        // the sweep (FP32 d=6 n=4: 34.2 against 36.2 us flushing first).
-        if constexpr (kCoefLds) flush_if_new(e);
-        lds_barrier();  // LDS free: the previous entry's last phase has been read by everyone
-        Lds<T, PL>::store_input(lds, pre, t);
-        if constexpr (kCoefLds) Coef<T, PL>::store(coef, pre_coef, t);
-        lds_barrier();
-        if (e + 1 < e1)
+        using LF = LaneFactors<PL>;
+        int const lane = t & 63;
+        auto entry = [&](int e) { return mats + static_cast<size_t>(e < e1 ? e : e1 - 1) * PL::kD; };
+        LF now, then;
+        typename LF::Next next;
+        next.address(entry(e0), lane);
+        next.load(now.a, stride, lane);
+        next.address(entry(e0 + 1), lane);
+        load_input<T, PL>(in[e0], pre, t);
+        for (int e = e0; e < e1; ++e)
         {
-            load_input<T, PL>(in[e + 1], pre, t);
-            if constexpr (kCoefLds)
-                Coef<T, PL>::load(mats + static_cast<size_t>(e + 1) * PL::kD, stride, pre_coef, t);
-        }
-        Lds<T, PL>::template read<0>(lds, v, t);
-        run_phases<T, PL, 0, true>(lds, v, mats + static_cast<size_t>(e) * PL::kD, stride, coef, t);
-        if constexpr (!kCoefLds) flush_if_new(e);
+            lds_barrier();  // LDS free: the previous entry's last phase has been read by everyone
+            Lds<T, PL>::store_input(lds, pre, t);
+            lds_barrier();
+            next.load(then.a, stride, lane);
+            next.address(entry(e + 2), lane);
+            if (e + 1 < e1) load_input<T, PL>(in[e + 1], pre, t);
+            Lds<T, PL>::template read<0>(lds, v, t);
+            run_phases<T, PL, 0, true>(lds, v, nullptr, stride, now, t);
+            flush_if_new(e);
 #pragma unroll
-        for (int j = 0; j < PL::R; ++j) acc[j] += v[j];
+            for (int j = 0; j < PL::R; ++j) acc[j] += v[j];
+            now = then;
+        }
+        if constexpr (ORDERED)
+            flush_piece<T, PL>(cur, acc, t, out, ws, nb, ps, e1);
+        else
+            flush<T, PL>(cur, acc, t);
+        return;
     }
-    if constexpr (ORDERED)
-        flush_piece<T, PL>(cur, acc, t, out, ws, nb, ps, e1);
     else
-        flush<T, PL>(cur, acc, t);
+    {
+        load_input<T, PL>(in[e0], pre, t);
+        if constexpr (kCoefLds) Coef<T, PL>::load(mats + static_cast<size_t>(e0) * PL::kD, stride, pre_coef, t);
+
+        for (int e = e0; e < e1; ++e)
+        {
+            // With factors staged in LDS the previous run is flushed before the sweep, not after it: with the
+            // branch between the last phase and the accumulation, the compiler issued that phase's coefficient
+            // reads (64 values for n = 8 FP64) above the branch and its FMAs below, holding all of them live
+            // (220 VGPRs; 120 flushing first; d=4 n=8: 236 -> 210 us per launch). The other plans flush after
+            // the sweep (FP32 d=6 n=4: 34.2 against 36.2 us flushing first).
+            if constexpr (kCoefLds) flush_if_new(e);
+            lds_barrier();  // LDS free: the previous entry's last phase has been read by everyone
+            Lds<T, PL>::store_input(lds, pre, t);
+            if constexpr (kCoefLds) Coef<T, PL>::store(coef, pre_coef, t);
+            lds_barrier();
+            if (e + 1 < e1)
+            {
+                load_input<T, PL>(in[e + 1], pre, t);
+                if constexpr (kCoefLds)
+                    Coef<T, PL>::load(mats + static_cast<size_t>(e + 1) * PL::kD, stride, pre_coef, t);
+            }
+            Lds<T, PL>::template read<0>(lds, v, t);
+            run_phases<T, PL, 0, true>(lds, v, mats + static_cast<size_t>(e) * PL::kD, stride, coef, t);
+            if constexpr (!kCoefLds) flush_if_new(e);
+    #pragma unroll
+            for (int j = 0; j < PL::R; ++j) acc[j] += v[j];
+        }
+        if constexpr (ORDERED)
+            flush_piece<T, PL>(cur, acc, t, out, ws, nb, ps, e1);
+        else
+            flush<T, PL>(cur, acc, t);
+    }
 }
 
 // Several Kronecker terms per entry: output[e] += sum_t kron(A_{t,e,0..d-1}) input[e], t = 0..nterm-1, with
@@ -689,6 +817,25 @@ __global__ void __launch_bounds__(PL::P) __attribute__((amdgpu_waves_per_eu(2)))
     T pre[PL::R];
     T pre_coef[kCoefLds ? Coef<T, PL>::kPerThread : 1];
     T x0[PL::R], v[PL::R];
+    using LF = LaneFactors<PL>;  // FP32 only
+    int const lane = t & 63;
+    LF now, then;
+    typename LF::Next next;
+    int se = e0, st = 0;  // the sweep whose factor addresses are in `next`
+    auto advance = [&]() {
+        if (++st == nterm)
+        {
+            st = 0;
+            se = se + 1 < e1 ? se + 1 : se;
+        }
+    };
+    if constexpr (lane_factors<T, PL>())
+    {
+        next.address(factors(0, e0), lane);
+        next.load(now.a, stride, lane);
+        advance();
+        next.address(factors(st, se), lane);
+    }
     load_input<T, PL>(in[e0], pre, t);
     if constexpr (kCoefLds) Coef<T, PL>::load(factors(0, e0), stride, pre_coef, t);
     T *cur = out[e0];
@@ -705,10 +852,20 @@ __global__ void __launch_bounds__(PL::P) __attribute__((amdgpu_waves_per_eu(2)))
         Lds<T, PL>::store_input(lds, pre, t);
         if constexpr (kCoefLds) Coef<T, PL>::store(coef, pre_coef, t);
         lds_barrier();
+        auto following = [&]() {
+            if constexpr (lane_factors<T, PL>())
+            {
+                next.load(then.a, stride, lane);
+                advance();
+                next.address(factors(st, se), lane);
+            }
+        };
+        following();
         if (e + 1 < e1) load_input<T, PL>(in[e + 1], pre, t);
         Lds<T, PL>::template read<0>(lds, x0, t);
         for (int term = 0; term < nterm; ++term)
         {
+            if (term > 0) following();
             if constexpr (kCoefLds)
             {
                 if (term + 1 < nterm)
@@ -718,7 +875,13 @@ __global__ void __launch_bounds__(PL::P) __attribute__((amdgpu_waves_per_eu(2)))
             }
 #pragma unroll
             for (int j = 0; j < PL::R; ++j) v[j] = x0[j];
-            run_phases<T, PL, 0>(lds, v, factors(term, e), stride, coef, t);
+            if constexpr (lane_factors<T, PL>())
+            {
+                run_phases<T, PL, 0>(lds, v, nullptr, stride, now, t);
+                now = then;
+            }
+            else
+                run_phases<T, PL, 0>(lds, v, factors(term, e), stride, coef, t);
 #pragma unroll
             for (int j = 0; j < PL::R; ++j) acc[j] += v[j];
             if constexpr (kCoefLds)
