@@ -240,27 +240,34 @@ struct LaneFactors
         }
     };
 
+    // element k of fiber f in the register index, where the mode has stride S
+    static constexpr int place(int f, int k, int S) { return f / S * S * N + f % S + k * S; }
+
     // contract mode M, which has stride S in the register index
     template<int M, int R, int S>
     __device__ __forceinline__ void contract(float (&v)[R]) const
     {
-        constexpr int F = R / N;  // fibers of this lane
-        Quad y[F][H];
+        constexpr int F = R / N;          // fibers of this lane
+        constexpr int G = F < 4 ? F : 4;  // fibers at a time: enough independent chains, few registers beside v
 #pragma unroll
-        for (int f = 0; f < F; ++f)
+        for (int f0 = 0; f0 < F; f0 += G)
+        {
+            Quad y[G][H];
 #pragma unroll
-            for (int h = 0; h < H; ++h) y[f][h] = Quad{0.f, 0.f, 0.f, 0.f};
-        static_for<0, N * H>([&](auto step) {
-            constexpr int k = step.value / H, h = step.value % H, q = (M * H + h) * N + k;
+            for (int g = 0; g < G; ++g)
 #pragma unroll
-            for (int f = 0; f < F; ++f)
-                y[f][h] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[q / 16], v[f / S * S * N + f % S + k * S], y[f][h], 4,
-                                                             q % 16, 0);
-        });
+                for (int h = 0; h < H; ++h) y[g][h] = Quad{0.f, 0.f, 0.f, 0.f};
+            static_for<0, N * H>([&](auto step) {
+                constexpr int k = step.value / H, h = step.value % H, q = (M * H + h) * N + k;
 #pragma unroll
-        for (int f = 0; f < F; ++f)
+                for (int g = 0; g < G; ++g)
+                    y[g][h] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[q / 16], v[place(f0 + g, k, S)], y[g][h], 4, q % 16, 0);
+            });
 #pragma unroll
-            for (int r = 0; r < N; ++r) v[f / S * S * N + f % S + r * S] = y[f][r / 4][r % 4];
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int r = 0; r < N; ++r) v[place(f0 + g, r, S)] = y[g][r / 4][r % 4];
+        }
     }
 };
 

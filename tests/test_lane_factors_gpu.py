@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
-from helpers import shift_odd_inputs
+from helpers import accumulation_bound, shift_odd_inputs, terms_reference
 from kronmult993_amd import workloads as W
 from kronmult993_amd.device import DeviceBatch
 
@@ -45,3 +45,24 @@ def test_subnormal_and_special_values(gpu, d, n):
     x[int(b.in_off[7]) + 5] = np.inf
     x[int(b.in_off[9]) + 3] = np.nan
     _check(W.HostBatch(**{**b.__dict__, "mat_pool": mats, "in_pool": x}), gpu)
+
+
+@pytest.mark.parametrize("nb,terms", [(1, 2), (5, 1), (700, 1), (2047, 3), (2050, 2), (6147, 2)])
+def test_wavefront_per_entry(gpu, nb, terms):
+    """d=6 n=4: wavefronts with one entry, several and none; outputs that end inside a wavefront's run, with it, and
+    with a workgroup's, so that neighbours' sums are added in every combination."""
+    b = W.random_terms(450 + nb, 6, 4, nb, terms, stride=5, shared_factors=29, distinct=nb // 3 + 1, dtype=np.float32)
+
+    def run(c):
+        db = DeviceBatch(c, device=str(gpu))
+        db.run_terms() if terms > 1 else db.run()
+        return db.output()
+
+    own = np.tile(np.arange(nb, dtype=np.int64), terms)
+    u = shift_odd_inputs(W.HostBatch(**{**b.__dict__, "out_count": nb, "out_index": own, "out_init": None}))
+    assert np.array_equal(run(u), terms_reference(u, True))
+    for group in (1, 2, 3, 5, 16):  # consecutive entries per output
+        shared = np.tile(np.arange(nb, dtype=np.int64) // group, terms)
+        c = W.HostBatch(**{**b.__dict__, "out_count": (nb + group - 1) // group, "out_index": shared, "out_init": None})
+        err = np.abs(run(c).astype(np.float64) - oracle.kronmult(c).astype(np.float64))
+        assert float(np.max(err - accumulation_bound(c, np.finfo(np.float32).eps / 2))) <= 0.0, group
