@@ -539,7 +539,8 @@ struct NoHook
 // Wave priority raised over a phase's contraction (S_SETPRIO 1, back to 0 before the LDS exchange): the
 // arbiter then favours waves that are in their FMA chains over waves that are between barriers. Measured
 // in the one-term sweep (per launch): d=6 n=4 FP64 47.2 against 48.0 us, FP32 30.9 against 33.5 us;
-// d=4 n=8 FP32 149 against 186 us; d=3 n=8 FP32 9.4 against 9.6 us; the other FP32 plans unchanged.
+// d=4 n=8 FP32 149 against 186 us; d=3 n=8 FP32 9.4 against 9.6 us; the other FP32 plans unchanged (FP32 with
+// vector FMAs; with the products on the matrix cores d=6 n=4 is the same either way).
 // FP64 d=5 n=4 (53.5 against 53.1 us), FP64 d=4 n=8 (274 against 271 us) and the several-term sweep
 // (128.6 against 120.5 us per step) lost, so those keep the default priority.
 template<typename T, typename PL, bool PRIO>

@@ -1,5 +1,5 @@
-// kron_wave.hpp -- one wavefront per entry for small tensors (n^d <= 64 with 2 <= n <= 8, and a few shapes
-// of up to 256 elements; no counterpart in the reference, whose kernel gives every entry a workgroup of its
+// kron_wave.hpp -- one wavefront per entry for small tensors (n^d <= 64 with 2 <= n <= 8, and d=3 n=5, d=2
+// n=9, 10; no counterpart in the reference, whose kernel gives every entry a workgroup of its
 // own, kronmult_gpu/kronmult.cu:95-130).
 //
 // A workgroup is one wavefront and walks a run of consecutive entries. Lane l holds elements l + 64 j of
@@ -22,7 +22,7 @@ namespace kronwave
 
 constexpr int kLanes = 64;
 constexpr int kMaxD = 8;          // n >= 2 and n^d <= kMaxElems
-constexpr int kMaxElems = 256;    // elements per entry: at most 4 per lane
+constexpr int kMaxElems = 256;    // elements per entry (the shapes built: at most 125, two per lane)
 constexpr int kCoefPerLane = 2;   // d n^2 <= 128 for every one-element-per-lane shape
 constexpr int kMaxCoef = kCoefPerLane * kLanes;
 

@@ -15,6 +15,8 @@
 //     entries and accumulates same-output contributions in registers before one atomic flush;
 //   * block sweep (kron_block.hpp, kron_final.hpp) for the other shapes of the reference's grid above 200 elements:
 //     whole entries in LDS, larger vectors in one pass in LDS and one in registers;
+//   * one wavefront per entry: small tensors (kron_wave.hpp), whole fibers per lane (kron_wave_fiber.hpp), FP32 d=6 n=4
+//     with several terms (kron_wave_terms.hpp);
 //   * fiber sweep (any d, n <= 64): the n^d vector lives in LDS (<= 64 KiB) or, beyond that, in the
 //     caller's per-entry workspace; one workgroup per entry; shared outputs are accumulated with
 //     hardware FP64/FP32 atomics (global_atomic_add_f64/f32).
