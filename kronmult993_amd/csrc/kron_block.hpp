@@ -11,7 +11,8 @@
 // round trip and a barrier) and, beside it, HBM. Hence
 //   * the factors are read into scalar registers, one SGPR operand per multiply-add: as many columns as kColSgprs
 //     holds one mode ahead (before the barrier that orders the mode's values), the rest at their use. 4608 entries
-//     of d=5 n=5 FP64 57.7 -> 45.8 us together with the next item, of d=4 n=7 FP32 43 -> 30 us;
+//     of d=5 n=5 FP64 57.7 -> 45.8 us together with the next item, of d=4 n=7 FP32 43 -> 30 us. FP32 whole entries
+//     with one fiber per thread keep them in the lanes instead (LaneCols): 29.1 -> 24.7 us;
 //   * the next entry's factors are brought into the L2 one entry ahead (Touch): a cold factor costs the chain two
 //     trips to HBM per mode (d=5 n=5 FP64 57.7 -> 47.4 us alone, d=4 n=9 FP64 198 -> 127 us);
 //   * the next block's values are read into registers while this one is swept;
@@ -56,6 +57,12 @@ struct Block
     typedef T VU __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
 
     static constexpr int pa(int e) { return PAD == 0 ? e : e + PAD * (e / N); }
+    // between consecutive elements of a fiber
+    template<int ST>
+    static constexpr int step()
+    {
+        return ST == 1 ? 1 : ST + PAD * (ST / N);
+    }
 
     // ---- staging: granules c*P + t in registers, then in LDS; the last S % GR elements one by one
     V pre[CPT];
@@ -124,7 +131,7 @@ struct Block
     static __device__ __forceinline__ void contract(T const *lds, Cols const &cols, T const *A_generic, int stride,
                                                     int t, T (&y)[F][N])
     {
-        constexpr int STEP = ST == 1 ? 1 : ST + PAD * (ST / N);
+        constexpr int STEP = step<ST>();
         kronreg::constant_ptr<T> A = kronreg::as_constant(A_generic);
         T x[F][N];
 #pragma unroll
@@ -159,7 +166,7 @@ struct Block
         if constexpr (M > 0)
         {
             constexpr int ST = ipow(N, G - 1 - M);
-            constexpr int STEP = ST == 1 ? 1 : ST + PAD * (ST / N);
+            constexpr int STEP = step<ST>();
             T y[F][N];
             contract<ST>(lds, cols, A[M], stride, t, y);
             cols.load(A[M - 1], stride);
@@ -210,6 +217,97 @@ struct Touch
     }
 };
 
+// FP32: the factors of an entry in the lanes and the products on the matrix cores, as LaneFactors (kron_reg.hpp), for
+// any n <= 10: a factor is H = ceil(n / 4) x n blocks of four rows of one column, sixteen to a register; rows past n repeat
+// the last one and their results are dropped. The values of the next entry are loaded during this one, from addresses
+// read one entry earlier.
+//
+// Taken where a thread has one fiber. Against FMA chains with the factor columns in scalar registers, 200 / 1500 / 6000
+// entries in us: d=4 n=7 5.6 / 12.3 / 31.0 -> 5.0 / 11.3 / 24.9, d=5 n=5 5.9 / 14.9 / 38.6 -> 5.5 / 14.5 / 34.6, d=4 n=6
+// 16.3 -> 14.9 (6000), n=9 79 -> 67, n=10 138 -> 113, d=3 n=9 14.7 -> 12.4, n=10 18.1 -> 14.2. With two and four fibers
+// the results' registers cost wavefronts (d=5 n=6 79 -> 89, d=6 n=5 220 -> 267); n = 3 gains nothing (11.5, 11.6).
+template<typename T, int N, int D, int P>
+constexpr bool lane_factors()
+{
+    return sizeof(T) == 4 && N > 4 && Block<T, N, D, 1, P>::F == 1;
+}
+
+template<typename B, int N, int D>
+struct LaneCols
+{
+    static constexpr int H = (N + 3) / 4, V = (H * N + 15) / 16;
+    float a[D][V];
+
+    __device__ __forceinline__ void load(float const *const (&A)[D], int stride, int lane)
+    {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+        {
+            int const q = i * 16 + (lane >> 2) < H * N ? i * 16 + (lane >> 2) : H * N - 1;
+            int const row = 4 * (q / N) + (lane & 3);
+            int const off = (row < N ? row : N - 1) + q % N * stride;
+#pragma unroll
+            for (int m = 0; m < D; ++m) a[m][i] = kronreg::as_global(A[m])[off];
+        }
+    }
+
+    // y = factor M times the thread's fibers
+    template<int M>
+    __device__ __forceinline__ void contract(float const *lds, int t, float (&y)[B::F][N]) const
+    {
+        constexpr int ST = ipow(N, D - 1 - M);
+        constexpr int STEP = B::template step<ST>();
+        float x[B::F][N];
+        kronreg::Quad z[B::F][H];
+#pragma unroll
+        for (int i = 0; i < B::F; ++i)
+        {
+            float const *p = lds + B::pa(B::template fiber<ST>(t, i));
+#pragma unroll
+            for (int k = 0; k < N; ++k) x[i][k] = p[k * STEP];
+#pragma unroll
+            for (int h = 0; h < H; ++h) z[i][h] = kronreg::Quad{0.f, 0.f, 0.f, 0.f};
+        }
+        kronreg::static_for<0, N * H>([&](auto s) {
+            constexpr int k = s.value / H, h = s.value % H, q = h * N + k;
+#pragma unroll
+            for (int i = 0; i < B::F; ++i)
+                z[i][h] = __builtin_amdgcn_mfma_f32_4x4x1f32(a[M][q / 16], x[i][k], z[i][h], 4, q % 16, 0);
+        });
+        // the matrix instruction takes every lane: it stays above the branch on active threads
+#pragma unroll
+        for (int i = 0; i < B::F; ++i)
+#pragma unroll
+            for (int r = 0; r < N; ++r)
+            {
+                y[i][r] = z[i][r / 4][r % 4];
+                asm volatile("" : "+v"(y[i][r]));
+            }
+    }
+
+    template<int M>
+    __device__ __forceinline__ void inner_modes(float *lds, int t) const
+    {
+        if constexpr (M > 0)
+        {
+            constexpr int ST = ipow(N, D - 1 - M);
+            constexpr int STEP = B::template step<ST>();
+            float y[B::F][N];
+            contract<M>(lds, t, y);
+#pragma unroll
+            for (int i = 0; i < B::F; ++i)
+            {
+                float *p = lds + B::pa(B::template fiber<ST>(t, i));
+                if (B::active(t, i))
+#pragma unroll
+                    for (int r = 0; r < N; ++r) p[r * STEP] = y[i][r];
+            }
+            kronreg::lds_barrier();
+            inner_modes<M - 1>(lds, t);
+        }
+    }
+};
+
 // Whole entries of n^D elements. A workgroup walks a run of epw entries and keeps the sum of consecutive entries with
 // one output in registers, in the layout of mode 0's fibers (coalesced).
 template<typename T, int N, int D, int P>
@@ -245,43 +343,86 @@ __global__ void __launch_bounds__(P)
         }
     };
     int const last = e1 - 1;
-    Touch<T, N, D, P> touch;
-    touch.init(mats, e0 < last ? e0 + 1 : last, t);
-    b.load(in[e0], t);
-    T const *A[D];
-#pragma unroll
-    for (int m = 0; m < D; ++m) A[m] = mats[static_cast<size_t>(e0) * D + m];
-    typename B::Cols cols;
-    cols.load(A[D - 1], stride);
-    for (int e = e0; e < e1; ++e)
+    if constexpr (lane_factors<T, N, D, P>())
     {
-        T *const dst = out[e];
-        if (dst != cur)
+        using LC = LaneCols<B, N, D>;
+        int const lane = t & 63;
+        T const *A[D];
+        auto address = [&](int e) {
+#pragma unroll
+            for (int m = 0; m < D; ++m) A[m] = mats[static_cast<size_t>(e < last ? e : last) * D + m];
+        };
+        LC now, then;
+        address(e0);
+        now.load(A, stride, lane);
+        address(e0 + 1);
+        b.load(in[e0], t);
+        for (int e = e0; e < e1; ++e)
         {
-            flush();
-            cur = dst;
+            T *const dst = out[e];
+            if (dst != cur)
+            {
+                flush();
+                cur = dst;
+            }
+            kronreg::lds_barrier();  // LDS free: every thread has read mode 0's fibers
+            b.store(lds, t);
+            kronreg::lds_barrier();
+            then.load(A, stride, lane);
+            address(e + 2);
+            if (e < last) b.load(in[e + 1], t);
+            now.template inner_modes<D - 1>(lds, t);
+            T y[B::F][N];
+            now.template contract<0>(lds, t, y);
+#pragma unroll
+            for (int i = 0; i < B::F; ++i)
+#pragma unroll
+                for (int r = 0; r < N; ++r) acc[i][r] += y[i][r];
+            now = then;
         }
-        kronreg::lds_barrier();  // LDS free: every thread has read mode 0's fibers
-        b.store(lds, t);
-        kronreg::lds_barrier();
-        int const en = e < last ? e + 1 : last;
-        T const *An[D];
-#pragma unroll
-        for (int m = 0; m < D; ++m) An[m] = mats[static_cast<size_t>(en) * D + m];
-        touch.next(mats, en < last ? en + 1 : last, stride, t);
-        if (e < last) b.load(in[en], t);
-        B::template inner_modes<D - 1>(lds, cols, A, stride, t);
-        T y[B::F][N];
-        B::template contract<ST>(lds, cols, A[0], stride, t, y);
-        cols.load(An[D - 1], stride);
-#pragma unroll
-        for (int i = 0; i < B::F; ++i)
-#pragma unroll
-            for (int r = 0; r < N; ++r) acc[i][r] += y[i][r];
-#pragma unroll
-        for (int m = 0; m < D; ++m) A[m] = An[m];
+        flush();
+        return;
     }
-    flush();
+    else
+    {
+        Touch<T, N, D, P> touch;
+        touch.init(mats, e0 < last ? e0 + 1 : last, t);
+        b.load(in[e0], t);
+        T const *A[D];
+#pragma unroll
+        for (int m = 0; m < D; ++m) A[m] = mats[static_cast<size_t>(e0) * D + m];
+        typename B::Cols cols;
+        cols.load(A[D - 1], stride);
+        for (int e = e0; e < e1; ++e)
+        {
+            T *const dst = out[e];
+            if (dst != cur)
+            {
+                flush();
+                cur = dst;
+            }
+            kronreg::lds_barrier();  // LDS free: every thread has read mode 0's fibers
+            b.store(lds, t);
+            kronreg::lds_barrier();
+            int const en = e < last ? e + 1 : last;
+            T const *An[D];
+#pragma unroll
+            for (int m = 0; m < D; ++m) An[m] = mats[static_cast<size_t>(en) * D + m];
+            touch.next(mats, en < last ? en + 1 : last, stride, t);
+            if (e < last) b.load(in[en], t);
+            B::template inner_modes<D - 1>(lds, cols, A, stride, t);
+            T y[B::F][N];
+            B::template contract<ST>(lds, cols, A[0], stride, t, y);
+            cols.load(An[D - 1], stride);
+#pragma unroll
+            for (int i = 0; i < B::F; ++i)
+#pragma unroll
+                for (int r = 0; r < N; ++r) acc[i][r] += y[i][r];
+#pragma unroll
+            for (int m = 0; m < D; ++m) A[m] = An[m];
+        }
+        flush();
+    }
 }
 
 // The fastest G modes of every entry: block s of entry e from in[e] to ws[e] (`items` blocks, per_entry of them in an

@@ -47,6 +47,20 @@ def test_subnormal_and_special_values(gpu, d, n):
     _check(W.HostBatch(**{**b.__dict__, "mat_pool": mats, "in_pool": x}), gpu)
 
 
+@pytest.mark.parametrize("d,n", [(3, 9), (3, 10), (4, 6), (4, 7), (4, 9), (4, 10), (5, 5)])
+def test_whole_entries(gpu, d, n):
+    """n not a multiple of four: the block sweep's rows past n, runs of one, two and more entries, special values."""
+    for nb in (1, 3, 1301):
+        b = W.random_case(470 + 7 * d + n, d, n, nb, stride=n + d % 3, shared_factors=23, distinct=nb // 3 + 1,
+                          dtype=np.float32)
+        _check(shift_odd_inputs(_own_outputs(b)), gpu)
+    b = _own_outputs(W.random_case(480 + 7 * d + n, d, n, 7, dtype=np.float32))
+    x = (b.in_pool * np.float32(1e-39)).astype(np.float32)
+    x[int(b.in_off[3]) + 5] = np.inf
+    x[int(b.in_off[5]) + 3] = np.nan
+    _check(W.HostBatch(**{**b.__dict__, "in_pool": x}), gpu)
+
+
 @pytest.mark.parametrize("nb,terms", [(1, 2), (5, 1), (700, 1), (2047, 3), (2050, 2), (6147, 2)])
 def test_wavefront_per_entry(gpu, nb, terms):
     """d=6 n=4: wavefronts with one entry, several and none; outputs that end inside a wavefront's run, with it, and
