@@ -73,6 +73,11 @@ struct Adj
         T const *p = lds + B::pa(B::template fiber<st(M)>(t, 0));
 #pragma unroll
         for (int k = 0; k < N; ++k) v[k] = p[k * step(M)];
+        // a thread past the last fiber holds zeros, in x and in the cotangent: its products add nothing, whatever the
+        // values of the fiber that it repeats (0 times infinity would not be 0)
+        if (!B::active(t, 0))
+#pragma unroll
+            for (int k = 0; k < N; ++k) v[k] = T(0);
     }
     template<int M>
     static __device__ __forceinline__ void write(T *lds, int t, T const (&v)[N])
@@ -337,13 +342,7 @@ __global__ void __launch_bounds__(P)
         // modes M .. D-1 of the cotangent
         auto hchain = [&](auto self, auto mc) -> void {
             constexpr int M = decltype(mc)::value;
-            if constexpr (M > 0)
-            {
-                A::template read<M>(lds, t, h);
-                if (!B::active(t, 0))
-#pragma unroll
-                    for (int r = 0; r < N; ++r) h[r] = T(0);
-            }
+            if constexpr (M > 0) A::template read<M>(lds, t, h);
             if (want_mats)
             {
                 if constexpr (M == 0)
