@@ -333,8 +333,8 @@ __global__ void __launch_bounds__(kThreads)
                         T *const *__restrict__ gmats, T *const *__restrict__ ws)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    int const e0 = kronreg::xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
+    int const e0 = kronreg::xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     bool const wave0 = threadIdx.x < 64;
     T dacc[kRunD][4];
     T *dptr[kRunD];

@@ -319,8 +319,8 @@ __global__ void __launch_bounds__(P)
     __shared__ __attribute__((aligned(16))) T lds[B::LDS];
     constexpr int ST = ipow(N, D - 1);
     int const t = threadIdx.x;
-    int const e0 = kronreg::xcd_run_index() * epw;
-    int const e1 = (nb - e0 > epw) ? e0 + epw : nb;
+    int const e0 = kronreg::xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     if (e0 >= e1) return;
     B b;
     T acc[B::F][N];
@@ -436,8 +436,8 @@ __global__ void __launch_bounds__(P)
     __shared__ __attribute__((aligned(16))) T lds[B::LDS];
     constexpr int ST = ipow(N, G - 1);
     int const t = threadIdx.x;
-    int const w0 = kronreg::xcd_run_index() * run;
-    int const w1 = (items - w0 > run) ? w0 + run : items;
+    int const w0 = kronreg::xcd_run_begin(run, items);
+    int const w1 = kronruns::end(w0, run, items);
     if (w0 >= w1) return;
     B b;
     int e = w0 / per_entry, s = w0 - e * per_entry;

@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(p
         while (gi + 1 < table.count && tile >= table.tile_start[gi + 1]) ++gi;
         GroupDesc<T> const &G = table.g[gi];
         int const e_begin = (tile - table.tile_start[gi]) * G.epw;
-        int const e_end = e_begin + G.epw < G.nb ? e_begin + G.epw : G.nb;
+        int const e_end = kronruns::end(e_begin, G.epw, G.nb);
         // wave paths: each wavefront sweeps a contiguous quarter of the tile on its own
         int const w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kronwave::kLanes);
         int const lane = static_cast<int>(threadIdx.x) & (kronwave::kLanes - 1);

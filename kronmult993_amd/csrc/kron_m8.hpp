@@ -169,8 +169,8 @@ __global__ void __launch_bounds__(M8Plan<D>::P)
     double *const coef0 = lds + (k2 ? 2 : 1) * PL::SIZE;
     int const t = threadIdx.x;
     int const lane = t & 63;
-    int const e0 = kronreg::xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
+    int const e0 = kronreg::xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     if (e0 >= e1) return;
 
     unsigned const in_base = static_cast<unsigned>(SwizzleIn::phys(2 * t) * 8);  // granule t of each block

@@ -121,8 +121,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
     int const t = threadIdx.x;
     int const w = t >> 6, lane = t & 63;
     int const kb = lane >> 4, jb = (lane >> 2) & 3, s = lane & 3;
-    int const e0 = kronreg::xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
+    int const e0 = kronreg::xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     if (e0 >= e1) return;
 
     // the factor operand of this lane for every mode: A_m[i = lane & 3][k = lane >> 4]

@@ -29,14 +29,14 @@ struct Walk
     {
         while (left > 0)
         {
-            int const k = c + r * period;
+            unsigned const k = static_cast<unsigned>(c) + static_cast<unsigned>(r) * static_cast<unsigned>(period);
             --left;
             if (++r == rows)
             {
                 r = 0;
                 ++c;
             }
-            if (k < nb) return k;
+            if (k < static_cast<unsigned>(nb)) return static_cast<int>(k);
         }
         return -1;
     }

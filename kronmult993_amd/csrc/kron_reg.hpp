@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "kron_plan.hpp"
+#include "kron_runs.hpp"
 
 namespace kronreg
 {
@@ -619,6 +620,11 @@ __device__ __forceinline__ int xcd_run_index()
     int const per_xcd = gridDim.x >> 3;
     return (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
 }
+// The workgroup's first entry, nb if its run lies past the batch
+__device__ __forceinline__ int xcd_run_begin(long epw, int nb)
+{
+    return kronruns::begin(xcd_run_index(), epw, nb);
+}
 
 
 // S_WAITCNT immediate for vmcnt(0) with the export and LDS counters left alone (gfx9 encoding: vmcnt in
@@ -657,8 +663,8 @@ __global__ void __launch_bounds__(PL::P) __attribute__((amdgpu_waves_per_eu(min_
     __shared__ __attribute__((aligned(16))) T lds[PL::SIZE + kCoefSlots];
     T *coef = lds + PL::SIZE;
     int const t = threadIdx.x;
-    int const e0 = xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
+    int const e0 = xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     if (e0 >= e1) return;
 
     T acc[PL::R];
@@ -814,8 +820,8 @@ __global__ void __launch_bounds__(PL::P) __attribute__((amdgpu_waves_per_eu(2)))
     __shared__ __attribute__((aligned(16))) T lds[PL::SIZE + kCoefSlots];
     T *coef = lds + PL::SIZE;
     int const t = threadIdx.x;
-    int const e0 = xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
+    int const e0 = xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     if (e0 >= e1) return;
     auto factors = [&](int term, int e) { return mats + (static_cast<size_t>(term) * nb + e) * PL::kD; };
 

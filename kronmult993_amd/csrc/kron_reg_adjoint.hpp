@@ -387,8 +387,8 @@ __global__ void __launch_bounds__(PL::P)
     constexpr int R = S::R, P = S::P, D = S::D;
     __shared__ __attribute__((aligned(16))) T lds[S::lds_elems(STORE)];
     int const t = threadIdx.x;
-    int const e0 = kronreg::xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
+    int const e0 = kronreg::xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     if (e0 >= e1) return;
     bool const want_mats = gmats != nullptr;
     bool const want_input = gin != nullptr;

@@ -294,8 +294,8 @@ __global__ void __launch_bounds__(PL::P) __attribute__((amdgpu_waves_per_eu(3)))
     __shared__ __attribute__((aligned(16))) double lds[PL::SIZE + table_bytes<PL>() / 8];
     unsigned char *const tabs = reinterpret_cast<unsigned char *>(lds + PL::SIZE);
     int const t = threadIdx.x;
-    int const e0 = kronreg::xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
+    int const e0 = kronreg::xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     if (e0 >= e1) return;
     auto tab_of = [&](int e) { return tabs + (e & 1) * (PL::kD * kFactorBytes); };
 

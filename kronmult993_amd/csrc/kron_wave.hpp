@@ -178,8 +178,8 @@ __global__ void __launch_bounds__(kLanes)
                      T *const *__restrict__ out)
 {
     __shared__ T rows[wave_lds<D, N>()];
-    int const e0 = kronreg::xcd_run_index() * epw;
-    int const e1 = (e0 + epw < nb) ? e0 + epw : nb;
+    int const e0 = kronreg::xcd_run_begin(epw, nb);
+    int const e1 = kronruns::end(e0, epw, nb);
     if (e0 >= e1) return;
     constexpr int XS = (wave_size<D, N>() + kLanes - 1) / kLanes * kLanes;
     wave_run<T, D, N>(e0, e1, mats, stride, in, out, rows, rows + XS, static_cast<int>(threadIdx.x));

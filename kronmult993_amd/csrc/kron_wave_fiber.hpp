@@ -225,8 +225,8 @@ struct FiberWave
                                                  T const *const *__restrict__ in, T *const *__restrict__ out, T *rows,
                                                  T **last, int wave, int lane)
     {
-        int const e0 = g1 - g0 > wave * epw ? g0 + wave * epw : g1;
-        int const e1 = g1 - e0 > epw ? e0 + epw : g1;
+        int const e0 = g0 + kronruns::begin(wave, epw, g1 - g0);
+        int const e1 = kronruns::end(e0, epw, g1);
         T acc[F][N];
 #pragma unroll
         for (int i = 0; i < F; ++i)
@@ -246,9 +246,10 @@ __global__ void __launch_bounds__(kLanes *kWaves)
     using FW = FiberWave<T, D, N>;
     __shared__ __attribute__((aligned(16))) T rows[kWaves * FW::LDS];
     __shared__ T *last[kWaves];
-    int const g0 = kronreg::xcd_run_index() * epw * kWaves;
+    long const per_group = static_cast<long>(epw) * kWaves;
+    int const g0 = kronreg::xcd_run_begin(per_group, nb);
     if (g0 >= nb) return;
-    int const g1 = nb - g0 > epw * kWaves ? g0 + epw * kWaves : nb;
+    int const g1 = kronruns::end(g0, per_group, nb);
     int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     FW::group(g0, g1, epw, mats, stride, in, out, rows, last, wave, static_cast<int>(threadIdx.x & 63));
 }

@@ -66,11 +66,11 @@ __global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_e
     __shared__ float *last[kWaves];
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    long const first = static_cast<long>(kronreg::xcd_run_index()) * kWaves * run;
+    int const first = kronreg::xcd_run_begin(static_cast<long>(run) * kWaves, nb);
     if (first >= nb) return;
     float *const lds = all[wave];
-    int const e0 = static_cast<int>(first + wave * run < nb ? first + wave * run : nb);
-    int const e1 = nb - e0 > run ? e0 + run : nb;
+    int const e0 = first + kronruns::begin(wave, run, nb - first);
+    int const e1 = kronruns::end(e0, run, nb);
 
     float acc[64];
 #pragma unroll

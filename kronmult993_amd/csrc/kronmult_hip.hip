@@ -352,7 +352,7 @@ hipError_t wave_terms_launch(Shape const &s, int nterm, Launch &L, float const *
     L.epw = per_wave * kronwaveterms::kWaves;
     L.lds = sizeof(float) * kronwaveterms::kWaves * kronwaveterms::PL::SIZE;
     if (!run) L.resident = resident_per_cu(kronwaveterms::kron_wave_terms_kernel, L.block, 0);
-    long const groups = (s.nb + L.epw - 1) / L.epw;
+    long const groups = kronruns::count(s.nb, L.epw);
     L.grid = (groups + 7) / 8 * 8;  // surplus workgroups exit at once
     if (!run) return hipSuccess;
     hipLaunchKernelGGL(kronwaveterms::kron_wave_terms_kernel, dim3(static_cast<unsigned>(L.grid)), dim3(L.block), 0,
@@ -399,7 +399,7 @@ hipError_t reg_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L, T 
     int epw = tu.entries_per_workgroup > 0 ? tu.entries_per_workgroup : static_cast<int>((s.nb + slots - 1) / slots);
     if (epw < 1) epw = 1;
     L.epw = epw;
-    long const runs = (s.nb + epw - 1) / epw;
+    long const runs = kronruns::count(s.nb, epw);
     L.grid = (runs + 7) / 8 * 8;  // surplus runs exit at once
     if (!run) return hipSuccess;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(L.grid)), dim3(block), 0, stream, s.nb, epw, mats,
@@ -424,7 +424,7 @@ hipError_t mfma_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L, d
     int epw = tu.entries_per_workgroup > 0 ? tu.entries_per_workgroup : static_cast<int>((s.nb + slots - 1) / slots);
     if (epw < 1) epw = 1;
     L.epw = epw;
-    long const runs = (s.nb + epw - 1) / epw;
+    long const runs = kronruns::count(s.nb, epw);
     L.grid = (runs + 7) / 8 * 8;
     if (!run) return hipSuccess;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(L.grid)), dim3(256), 0, stream, s.nb, epw, mats, s.stride,
@@ -693,7 +693,7 @@ hipError_t wave_fiber_launch(Shape const &s, int family, int entries_per_workgro
     L.block = kronwave::kLanes * kronwave::kWaves;
     long const per_wg = static_cast<long>(epw) * kronwave::kWaves;
     L.epw = static_cast<int>(std::min<long>(per_wg, INT_MAX));
-    L.grid = ((s.nb + per_wg - 1) / per_wg + 7) / 8 * 8;  // whole XCD stripes; surplus workgroups exit at once
+    L.grid = (kronruns::count(s.nb, per_wg) + 7) / 8 * 8;  // whole XCD stripes; surplus workgroups exit at once
 #define KRON_WAVE_FIBER_LAUNCH(D, N)                                                                                   \
     if (s.d == D && s.n == N)                                                                                          \
     {                                                                                                                  \
@@ -736,7 +736,7 @@ hipError_t block_launch_dn(Shape const &s, Launch &L, T const *const *mats, T co
     long const slots = static_cast<long>(device_cu_count()) * block_workgroups_per_cu(P, sizeof(T));
     L.epw = static_cast<int>((s.nb + slots - 1) / slots);
     if (L.epw < 1) L.epw = 1;
-    long const runs = (static_cast<long>(s.nb) + L.epw - 1) / L.epw;
+    long const runs = kronruns::count(s.nb, L.epw);
     L.grid = (runs + 7) / 8 * 8;  // whole XCD stripes; surplus runs exit at once
     if (!run) return hipSuccess;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(L.grid)), dim3(P), 0, stream, s.nb, L.epw, mats, s.stride, in,
@@ -943,7 +943,7 @@ hipError_t packed_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L,
     size_t const lds = fill_group<T>(s, mats, in, out, ept, table.g[0]);
     table.count = 1;
     table.tile_start[0] = 0;
-    table.tiles = (s.nb + table.g[0].epw - 1) / table.g[0].epw;
+    table.tiles = static_cast<int>(kronruns::count(s.nb, table.g[0].epw));
     table.tile_start[1] = table.tiles;
     int const per_cu = tu.workgroups_per_cu > 0 ? tu.workgroups_per_cu : kPackedWorkgroupsPerCu;
     long grid = static_cast<long>(device_cu_count()) * per_cu;
@@ -992,7 +992,7 @@ hipError_t wave_launch_dn(Shape const &s, kronmult_tuning_t const &tu, Launch &L
     }
     if (epw < 1) epw = 1;
     L.epw = static_cast<int>(epw);
-    long const runs = (s.nb + epw - 1) / epw;
+    long const runs = kronruns::count(s.nb, epw);
     L.grid = (runs + 7) / 8 * 8;  // whole XCD stripes; surplus runs exit at once
     if (L.grid > INT_MAX) return hipErrorInvalidValue;
     if (!run || s.nb == 0) return hipSuccess;
@@ -1047,7 +1047,7 @@ hipError_t reduce_pieces(Shape const &s, Launch const &L, T *const *out, T *cons
     using namespace kronordered;
     bool const all = L.workspace && use_passes<T>(s);
     int const epw = all ? 1 : L.epw;
-    long const ranges = (s.nb + epw - 1) / epw;
+    long const ranges = kronruns::count(s.nb, epw);
     long const chunks = (s.size + kReduceThreads * kReducePer - 1) / (kReduceThreads * kReducePer);
     long const gy = chunks < 65535 ? chunks : 65535;
     // about 1024 workgroups: ranges per workgroup from 1 to 256 (one per thread)
@@ -1114,7 +1114,7 @@ hipError_t reg_terms_launch(Shape const &s, int nterm, T const *const *mats, T c
     long const slots = static_cast<long>(device_cu_count()) * default_workgroups_per_cu(PL::P);
     int epw = static_cast<int>((s.nb + slots - 1) / slots);
     if (epw < 1) epw = 1;
-    long const runs = (s.nb + epw - 1) / epw;
+    long const runs = kronruns::count(s.nb, epw);
     long const grid = (runs + 7) / 8 * 8;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(PL::P), 0, stream, s.nb, nterm, epw, mats,
                        s.stride, in, out);
@@ -1289,7 +1289,7 @@ hipError_t reg_adjoint_launch(Shape const &s, RegAdjMode mode, T const *const *m
     long const slots = static_cast<long>(device_cu_count()) * per_cu;
     int epw = static_cast<int>((s.nb + slots - 1) / slots);
     if (epw < 1) epw = 1;
-    long const runs = (s.nb + epw - 1) / epw;
+    long const runs = kronruns::count(s.nb, epw);
     long const grid = (runs + 7) / 8 * 8;
     dim3 const g(static_cast<unsigned>(grid)), blk(PL::P);
     switch (mode)
@@ -1399,7 +1399,7 @@ hipError_t adjoint_launch_n(Shape const &s, AdjointPlan const &p, T const *const
     long const slots = static_cast<long>(device_cu_count()) * resident_per_cu(kernel, p.threads, p.lds);
     int epw = static_cast<int>((s.nb + slots - 1) / slots);
     if (epw < 1) epw = 1;
-    long const runs = (s.nb + epw - 1) / epw;
+    long const runs = kronruns::count(s.nb, epw);
     long const grid = (runs + 7) / 8 * 8;  // surplus workgroups exit at once
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(p.threads), p.lds, stream, s.nb, epw, s.d,
                        static_cast<int>(s.size), mats, s.stride, in, gout, gin, gmats, ws);
@@ -1541,7 +1541,7 @@ hipError_t kronmult_grouped_launch(GroupT const *groups, int count, kronmult_gro
         size_t const need = fill_group<T>(s, g.matrix_list_batched, const_cast<T const *const *>(g.input_batched),
                                           g.output_batched, g.entries_per_tile, D, true);
         table.tile_start[table.count] = tiles;
-        tiles += (s.nb + D.epw - 1) / D.epw;
+        tiles += static_cast<int>(kronruns::count(s.nb, D.epw));
         if (need > lds) lds = need;
         paths |= 1 << D.path;
         ++table.count;
@@ -1604,7 +1604,7 @@ hipError_t split_reg_launch(Shape const &s, double const *const *mats, double co
     long const slots = static_cast<long>(device_cu_count()) * per_cu;
     int epw = static_cast<int>((s.nb + slots - 1) / slots);
     if (epw < 1) epw = 1;
-    long const runs = (s.nb + epw - 1) / epw;
+    long const runs = kronruns::count(s.nb, epw);
     long const grid = (runs + 7) / 8 * 8;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(PL::P), 0, stream, s.nb, epw, mats,
                        s.stride, in, out);
@@ -1774,7 +1774,7 @@ hipError_t kronmult_ordered_noalloc(int d, int n, T const *const *mats, int stri
     if (nb == 0) return hipSuccess;
     if (mats == nullptr || in == nullptr || out == nullptr) return hipErrorInvalidValue;
     int const epw = (L.workspace && use_passes<T>(s)) ? 1 : L.epw;  // multi-pass: every entry is a piece
-    long const ranges = (static_cast<long>(nb) + epw - 1) / epw;
+    long const ranges = kronruns::count(nb, epw);
     long const slots = epw == 1 ? nb : 2 * ranges;
     size_t const ptr_bytes = (static_cast<size_t>(nb) * sizeof(T *) + 255) / 256 * 256;
     size_t const slot_bytes = static_cast<size_t>(s.size) * sizeof(T);
