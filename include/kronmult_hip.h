@@ -60,7 +60,8 @@ int kronmult_batched_f32_async(int matrix_count, int matrix_size, float const *c
  *                           n^(d-1) <= 64; the default for such shapes from 20 entries per CU on) or
  *                           _WAVE (one wavefront per entry: n^d <= 64 with 2 <= n <= 8, one element per lane,
  *                           and d=3 n=5; d=2 n=9,10 with two, and d=7,8 n=2; d=4,5 n=3; d=3 n=6 with
- *                           whole fibers per lane);
+ *                           whole fibers per lane: there a workgroup is four wavefronts, which take a quarter of
+ *                           its entries each);
  *   workgroups_per_cu:      workgroups to launch per compute unit (register, matrix, packed, wave families);
  *   entries_per_workgroup:  consecutive entries one workgroup walks (register, matrix, wave families), or
  *                           entries per tile (packed family).

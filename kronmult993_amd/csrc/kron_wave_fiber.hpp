@@ -238,6 +238,7 @@ struct FiberWave
     }
 };
 
+// epw: entries per workgroup, any number (its wavefronts take ceil(epw / kWaves) each, the last ones what is left)
 template<typename T, int D, int N>
 __global__ void __launch_bounds__(kLanes *kWaves)
     kron_wave_fiber_kernel(int nb, int epw, T const *const *__restrict__ mats, int stride,
@@ -246,12 +247,11 @@ __global__ void __launch_bounds__(kLanes *kWaves)
     using FW = FiberWave<T, D, N>;
     __shared__ __attribute__((aligned(16))) T rows[kWaves * FW::LDS];
     __shared__ T *last[kWaves];
-    long const per_group = static_cast<long>(epw) * kWaves;
-    int const g0 = kronreg::xcd_run_begin(per_group, nb);
+    int const g0 = kronreg::xcd_run_begin(epw, nb);
     if (g0 >= nb) return;
-    int const g1 = kronruns::end(g0, per_group, nb);
+    int const g1 = kronruns::end(g0, epw, nb);
     int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    FW::group(g0, g1, epw, mats, stride, in, out, rows, last, wave, static_cast<int>(threadIdx.x & 63));
+    FW::group(g0, g1, (epw - 1) / kWaves + 1, mats, stride, in, out, rows, last, wave, static_cast<int>(threadIdx.x & 63));
 }
 
 // Shapes whose single batches run here: of the wave family, of the fiber family, of the packed family's default.

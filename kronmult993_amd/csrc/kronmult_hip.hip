@@ -686,14 +686,13 @@ template<typename T>
 hipError_t wave_fiber_launch(Shape const &s, int family, int entries_per_workgroup, Launch &L, T const *const *mats,
                              T const *const *in, T *const *out, hipStream_t stream, bool run)
 {
-    int epw = s.nb > kWaveFiberEntriesPerCu * device_cu_count() ? 2 : 1;
-    if (entries_per_workgroup > 0) epw = (std::min(entries_per_workgroup, s.nb) - 1) / kronwave::kWaves + 1;
-    if (epw < 1) epw = 1;
+    int epw = kronwave::kWaves * (s.nb > kWaveFiberEntriesPerCu * device_cu_count() ? 2 : 1);
+    if (entries_per_workgroup > 0) epw = entries_per_workgroup;  // as asked for
     L.family = family;
     L.block = kronwave::kLanes * kronwave::kWaves;
-    long const per_wg = static_cast<long>(epw) * kronwave::kWaves;
-    L.epw = static_cast<int>(std::min<long>(per_wg, INT_MAX));
-    L.grid = (kronruns::count(s.nb, per_wg) + 7) / 8 * 8;  // whole XCD stripes; surplus workgroups exit at once
+    L.epw = epw;
+    L.grid = (kronruns::count(s.nb, epw) + 7) / 8 * 8;  // whole XCD stripes; surplus workgroups exit at once
+    if (L.grid > INT_MAX) return hipErrorInvalidValue;
 #define KRON_WAVE_FIBER_LAUNCH(D, N)                                                                                   \
     if (s.d == D && s.n == N)                                                                                          \
     {                                                                                                                  \
