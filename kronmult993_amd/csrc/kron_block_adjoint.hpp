@@ -172,7 +172,6 @@ __global__ void __launch_bounds__(P)
     __shared__ __attribute__((aligned(16))) T lds[(B::LDS + A::GR - 1) / A::GR * A::GR + A::COEF + A::CHAIN];
     __shared__ T red[A::RED];
     __shared__ T *gptr_shared[D];
-    __shared__ int first_shared;
     T *const coef = lds + (B::LDS + A::GR - 1) / A::GR * A::GR;
     T *const chain = coef + A::COEF + threadIdx.x;
     int const t = threadIdx.x, lane = t & 63;
@@ -180,7 +179,7 @@ __global__ void __launch_bounds__(P)
     bool const want_mats = gmats != nullptr, want_input = gin != nullptr;
     int const groups = static_cast<int>(gridDim.x);
     kronorder::Walk walk = kronorder::walk(
-        gin, nb, groups_shared < groups && kronorder::shared_gradients(gmats, nb, D) ? groups_shared : groups, &first_shared);
+        gin, nb, groups_shared < groups && kronorder::shared_gradients(gmats, nb, D) ? groups_shared : groups);
     int e = walk.next();
     if (e < 0) return;
     int en = walk.next();

@@ -2,22 +2,24 @@
 //
 // An entry's input gradient is n^d atomic adds unless the next entry of the run adds to the same vector. A batch listed
 // by output (as the forward call wants it) visits the inputs in turn: entry k and entry k + p share an input, their
-// neighbours do not. The workgroup therefore looks for the first entry after 0 that shares entry 0's gradient pointer,
-// p, and walks the entries k = c, c + p, c + 2p, ... column by column instead of k = 0, 1, 2, ...: every entry once in
-// either order, whatever the pointers are, and the sums of shared gradients in registers when they do repeat with that
-// period. d=6 n=4, 128 x 64 element pairs listed by output, FP64: 33.5 M atomic adds (about 200 G/s) become 2.1 M.
+// neighbours do not. The workgroup therefore guesses that p from a sample of the gradient pointers and walks the entries
+// k = c, c + p, c + 2p, ... column by column instead of k = 0, 1, 2, ...: every entry once in either order, whatever the
+// guess and the pointers are, and the sums of shared gradients in registers when they do repeat with that period.
+// d=6 n=4, 128 x 64 element pairs listed by output, FP64: 33.5 M atomic adds (about 200 G/s) become 2.1 M.
+//
+// Every workgroup guesses before its first entry, so the guess costs one round trip to memory: the first 256 pointers,
+// four per lane, and every 256th up to entry 4096, one per lane, compared in registers. Every distance from 1 to 4096
+// is 256 (j + 1) - i for one j < 16 and one i < 256, so in a batch with a period the smallest distance between equal
+// ones is the period. (A scan of the pointers from entry 1 on, a load per thread and step, was a chain of 16 to 64 round
+// trips: 9 to 12 us.)
 #pragma once
 
 #include <hip/hip_runtime.h>
-
-#include <climits>
 
 #include "kron_reg.hpp"
 
 namespace kronorder
 {
-
-constexpr int kScan = 4096;  // pointers looked at (16 loads per thread of a 256-thread workgroup)
 
 struct Walk
 {
@@ -55,28 +57,43 @@ __device__ __forceinline__ bool shared_gradients(T *const *gmats, int nb, int d)
     return __ballot(same) != 0;
 }
 
+// The smallest distance between equal ones of the sampled pointers, 1 if there are none (a guess: 32 bits of the
+// addresses are compared). Every wavefront finds the same answer.
+template<typename T>
+__device__ __forceinline__ int guess_period(T *const *ptr, int nb)
+{
+    constexpr int kHead = 256, kTail = 16;
+    int const lane = static_cast<int>(threadIdx.x) & 63;
+    auto bits = [](T *p) { return static_cast<unsigned>(reinterpret_cast<unsigned long long>(p) >> 2); };
+    unsigned head[kHead / 64];
+#pragma unroll
+    for (int c = 0; c < kHead / 64; ++c)
+        head[c] = bits(kronreg::as_global(ptr)[64 * c + lane < nb ? 64 * c + lane : 0]);
+    int const at = kHead * (lane % kTail + 1);
+    int const tail = static_cast<int>(bits(kronreg::as_global(ptr)[at < nb ? at : 0]));
+#pragma unroll 1
+    for (int j = 0; j < kTail && kHead * (j + 1) < nb; ++j)
+    {
+        unsigned const there = static_cast<unsigned>(__builtin_amdgcn_readlane(tail, j));
+        unsigned long long same[kHead / 64];
+#pragma unroll
+        for (int c = 0; c < kHead / 64; ++c) same[c] = __ballot(head[c] == there);
+        if ((same[0] | same[1] | same[2] | same[3]) == 0) continue;
+        int i = 0;  // the last of the head's equal to this one
+#pragma unroll
+        for (int c = 0; c < kHead / 64; ++c) i = same[c] != 0 ? 64 * c + 63 - __builtin_clzll(same[c]) : i;
+        return kHead * (j + 1) - i;
+    }
+    return 1;
+}
+
 // This workgroup's part of the batch, cut into `groups` (a multiple of 8, at most the grid) equal parts; the workgroups
 // past them get none. ptr may be null (natural order). Every thread calls it.
 template<typename T>
-__device__ __forceinline__ Walk walk(T *const *ptr, int nb, int groups, int *shared_min)
+__device__ __forceinline__ Walk walk(T *const *ptr, int nb, int groups)
 {
     int period = 1;
-    if (ptr != nullptr && nb > groups)
-    {
-        if (threadIdx.x == 0) *shared_min = INT_MAX;
-        __syncthreads();
-        T *const first = ptr[0];
-        int const limit = nb < kScan ? nb : kScan;
-        for (int q = 1 + static_cast<int>(threadIdx.x); q < limit; q += static_cast<int>(blockDim.x))
-            if (ptr[q] == first)
-            {
-                atomicMin(shared_min, q);
-                break;
-            }
-        __syncthreads();
-        int const p = __builtin_amdgcn_readfirstlane(*shared_min);
-        if (p != INT_MAX) period = p;
-    }
+    if (ptr != nullptr && nb > groups) period = guess_period(ptr, nb);
     Walk w;
     w.nb = nb;
     w.period = period;

@@ -231,12 +231,11 @@ __global__ void __launch_bounds__(kP)
     using L = kronreg::Lds<T, PL>;
     __shared__ __attribute__((aligned(16))) T lds[PL::SIZE * (2 + (kKeep4 ? 1 : 0))];
     __shared__ T red[6 * kWaves * 16];
-    __shared__ int first_shared;
     T *const x3buf = lds + PL::SIZE;
     T *const x4buf = lds + 2 * PL::SIZE;
     int const t = threadIdx.x;
     int const lane = t & 63;
-    kronorder::Walk walk = kronorder::walk(gin, nb, static_cast<int>(gridDim.x), &first_shared);
+    kronorder::Walk walk = kronorder::walk(gin, nb, static_cast<int>(gridDim.x));
     int e = walk.next();
     if (e < 0) return;
     bool const want_mats = gmats != nullptr;
