@@ -159,7 +159,9 @@ struct Adj
     static constexpr int kLaneShift = C0 == 64 ? 0 : C0 == 32 ? 1 : C0 == 16 ? 2 : C0 == 8 ? 3 : C0 == 4 ? 4 : 5;
 };
 
-template<typename T, int N, int D, int P>
+// MATS: with the factors' gradients. Without them the X chain, the products and their registers fall away, so more
+// workgroups are resident.
+template<typename T, int N, int D, int P, bool MATS>
 __global__ void __launch_bounds__(P)
     kron_block_adjoint_kernel(int nb, int groups_shared, T const *const *__restrict__ mats, int stride,
                               T const *const *__restrict__ in, T const *const *__restrict__ gout,
@@ -169,17 +171,18 @@ __global__ void __launch_bounds__(P)
     using B = typename A::B;
     constexpr bool kCoefLds = A::kCoefLds;
     constexpr int NN = A::NN;
-    __shared__ __attribute__((aligned(16))) T lds[(B::LDS + A::GR - 1) / A::GR * A::GR + A::COEF + A::CHAIN];
-    __shared__ T red[A::RED];
+    __shared__ __attribute__((aligned(16))) T lds[(B::LDS + A::GR - 1) / A::GR * A::GR + A::COEF + (MATS ? A::CHAIN : 0)];
+    __shared__ T red[MATS ? A::RED : 1];
     __shared__ T *gptr_shared[D];
     T *const coef = lds + (B::LDS + A::GR - 1) / A::GR * A::GR;
     T *const chain = coef + A::COEF + threadIdx.x;
     int const t = threadIdx.x, lane = t & 63;
     int const wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    bool const want_mats = gmats != nullptr, want_input = gin != nullptr;
+    constexpr bool want_mats = MATS;
+    bool const want_input = gin != nullptr;
     int const groups = static_cast<int>(gridDim.x);
     kronorder::Walk walk = kronorder::walk(
-        gin, nb, groups_shared < groups && kronorder::shared_gradients(gmats, nb, D) ? groups_shared : groups);
+        gin, nb, MATS && groups_shared < groups && kronorder::shared_gradients(gmats, nb, D) ? groups_shared : groups, B::S);
     int e = walk.next();
     if (e < 0) return;
     int en = walk.next();
@@ -342,7 +345,7 @@ __global__ void __launch_bounds__(P)
         auto hchain = [&](auto self, auto mc) -> void {
             constexpr int M = decltype(mc)::value;
             if constexpr (M > 0) A::template read<M>(lds, t, h);
-            if (want_mats)
+            if constexpr (want_mats)
             {
                 if constexpr (M == 0)
                     grad(mc, X0);
@@ -368,7 +371,7 @@ __global__ void __launch_bounds__(P)
             }
             if constexpr (M < D - 1) self(self, std::integral_constant<int, M + 1>());
         };
-        if (want_mats) xchain(xchain, std::integral_constant<int, D - 1>());
+        if constexpr (want_mats) xchain(xchain, std::integral_constant<int, D - 1>());
         hchain(hchain, std::integral_constant<int, 0>());
         if constexpr (!kCoefLds)
         {

@@ -87,13 +87,19 @@ __device__ __forceinline__ int guess_period(T *const *ptr, int nb)
     return 1;
 }
 
+// Small tensors with runs shorter than two entries stay in natural order: there is little to sum, and neighbours that
+// add to one vector at the same time wait for each other. As 64-input pairs, natural / by input: 2100 entries of d=5 n=4
+// FP32, 2048 workgroups, input gradient 11.4 / 17.9 us; 780 of d=6 n=4 FP32, 768 workgroups, both gradients 26.2 / 21.5,
+// 1100 of d=4 n=7 FP64, input gradient 25.4 / 21.6.
+constexpr int kAlwaysByInput = 2048;  // elements
+
 // This workgroup's part of the batch, cut into `groups` (a multiple of 8, at most the grid) equal parts; the workgroups
 // past them get none. ptr may be null (natural order). Every thread calls it.
 template<typename T>
-__device__ __forceinline__ Walk walk(T *const *ptr, int nb, int groups)
+__device__ __forceinline__ Walk walk(T *const *ptr, int nb, int groups, int size)
 {
     int period = 1;
-    if (ptr != nullptr && nb > groups) period = guess_period(ptr, nb);
+    if (ptr != nullptr && nb > groups && (size >= kAlwaysByInput || nb / 2 >= groups)) period = guess_period(ptr, nb);
     Walk w;
     w.nb = nb;
     w.period = period;

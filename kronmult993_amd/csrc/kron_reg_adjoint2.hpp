@@ -218,7 +218,8 @@ __device__ __forceinline__ void stage_wait()
     __builtin_amdgcn_s_waitcnt(kronreg::kWaitVmcnt0);  // this wavefront's LDS-DMA loads have landed
 }
 
-template<typename T>
+// MATS: with the factors' gradients (without them only the H chain is left, in 32 KB of LDS and half the registers)
+template<typename T, bool MATS>
 __global__ void __launch_bounds__(kP)
     kron_reg_adjoint2_kernel(int nb, T const *const *__restrict__ mats, int stride,
                              T const *const *__restrict__ in, T const *const *__restrict__ gout,
@@ -229,16 +230,16 @@ __global__ void __launch_bounds__(kP)
     constexpr bool kKeep4 = keep_x4<T>();
     constexpr bool kStageX = stage_x_ok<T>();
     using L = kronreg::Lds<T, PL>;
-    __shared__ __attribute__((aligned(16))) T lds[PL::SIZE * (2 + (kKeep4 ? 1 : 0))];
-    __shared__ T red[6 * kWaves * 16];
-    T *const x3buf = lds + PL::SIZE;
-    T *const x4buf = lds + 2 * PL::SIZE;
+    __shared__ __attribute__((aligned(16))) T lds[PL::SIZE * (MATS ? 2 + (kKeep4 ? 1 : 0) : 1)];
+    __shared__ T red[MATS ? 6 * kWaves * 16 : 1];
+    T *const x3buf = lds + (MATS ? 1 : 0) * PL::SIZE;
+    T *const x4buf = lds + (MATS ? 2 : 0) * PL::SIZE;
     int const t = threadIdx.x;
     int const lane = t & 63;
-    kronorder::Walk walk = kronorder::walk(gin, nb, static_cast<int>(gridDim.x));
+    kronorder::Walk walk = kronorder::walk(gin, nb, static_cast<int>(gridDim.x), PL::SIZE);
     int e = walk.next();
     if (e < 0) return;
-    bool const want_mats = gmats != nullptr;
+    constexpr bool want_mats = MATS;
     bool const want_input = gin != nullptr;
 
     T gacc[6], dxacc[kR];
@@ -285,7 +286,7 @@ __global__ void __launch_bounds__(kP)
             }
         };
         auto flush = [&]() {
-            if (pending != 0)
+            if (MATS && pending != 0)
                 flush_gradients(pending, gmats + static_cast<size_t>(pending_from) * 6, stride, red, t);
             pending = 0;
         };
@@ -298,7 +299,7 @@ __global__ void __launch_bounds__(kP)
         }
         else
             load_g(e, h);
-        if (want_mats)
+        if constexpr (want_mats)
         {
             if constexpr (kStageX)
             {
@@ -328,10 +329,10 @@ __global__ void __launch_bounds__(kP)
             grad(std::integral_constant<int, 0>(), v);
         }
         contract<T, 0, true>(h, A[0], stride);  // H_1
-        if (want_mats) grad(std::integral_constant<int, 1>(), xs);
+        if constexpr (want_mats) grad(std::integral_constant<int, 1>(), xs);
         contract<T, 1, true>(h, A[1], stride);  // H_2
         exchange<T, 2, 1>(lds, h, t, flush);  // dA_0, dA_1
-        if (want_mats)
+        if constexpr (want_mats)
         {
             restore(x3buf, v, t);
 #pragma unroll
@@ -340,7 +341,7 @@ __global__ void __launch_bounds__(kP)
             grad(std::integral_constant<int, 2>(), v);
         }
         contract<T, 2, true>(h, A[2], stride);  // H_3
-        if (want_mats) grad(std::integral_constant<int, 3>(), xs);
+        if constexpr (want_mats) grad(std::integral_constant<int, 3>(), xs);
         contract<T, 3, true>(h, A[3], stride);  // H_4
         exchange<T, 1, 0>(lds, h, t, [&]() {
             flush();  // dA_2, dA_3
@@ -348,7 +349,7 @@ __global__ void __launch_bounds__(kP)
             if constexpr (kStageX)
                 if (want_mats) stage_x(x3buf, in[e], t);
         });
-        if (want_mats)
+        if constexpr (want_mats)
         {
             if constexpr (kStageX)
             {
@@ -369,7 +370,7 @@ __global__ void __launch_bounds__(kP)
             grad(std::integral_constant<int, 4>(), v);
         }
         contract<T, 4, true>(h, A[4], stride);  // H_5
-        if (want_mats) grad(std::integral_constant<int, 5>(), xs);
+        if constexpr (want_mats) grad(std::integral_constant<int, 5>(), xs);
         if (want_input)
         {
             contract<T, 5, true>(h, A[5], stride);  // d x, phase-0 layout
@@ -388,7 +389,7 @@ __global__ void __launch_bounds__(kP)
             }
         }
     }
-    if (pending != 0)
+    if (MATS && pending != 0)
     {
         lds_barrier();
         flush_gradients(pending, gmats + static_cast<size_t>(pending_from) * 6, stride, red, t);

@@ -1315,12 +1315,17 @@ hipError_t reg_adjoint_launch(Shape const &s, RegAdjMode mode, T const *const *m
 // d = 6, n = 4: the two-modes-per-phase adjoint (kron_reg_adjoint2.hpp), one run per resident workgroup.
 // It serves AUTO (measured on the d=6 batch, listed by output: FP64 189 us, FP32 112 us, against 522 / 304 us for the
 // one-mode-per-phase kernel, which RECOMPUTE and STORE keep).
+// At most three workgroups per CU: the input gradient alone would leave room for six in FP32, whose shorter runs sum less
+// (as 64-input pairs, 3 / 6 per CU: 2100 entries 17.6 / 25.7 us, 8300 39.5 / 36.3).
+constexpr int kAdjoint2PerCu = 3;
+
 template<typename T>
 hipError_t adjoint2_launch(Shape const &s, T const *const *mats, T const *const *in, T const *const *gout,
                            T *const *gin, T *const *gmats, hipStream_t stream)
 {
-    auto kernel = kronregadj2::kron_reg_adjoint2_kernel<T>;
-    int const per_cu = resident_per_cu(kernel, kronregadj2::kP, 0);
+    auto kernel = gmats != nullptr ? kronregadj2::kron_reg_adjoint2_kernel<T, true>
+                                   : kronregadj2::kron_reg_adjoint2_kernel<T, false>;
+    int const per_cu = std::min(kAdjoint2PerCu, resident_per_cu(kernel, kronregadj2::kP, 0));
     long const grid = (std::min<long>(s.nb, static_cast<long>(device_cu_count()) * per_cu) + 7) / 8 * 8;
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kronregadj2::kP), 0, stream, s.nb, mats, s.stride, in,
                        gout, gin, gmats);
@@ -1338,7 +1343,8 @@ hipError_t block_adjoint_launch_dn(Shape const &s, T const *const *mats, T const
                                    T *const *gin, T *const *gmats, hipStream_t stream)
 {
     constexpr int P = kronblock::block_threads<N, D>();
-    auto kernel = kronblockadj::kron_block_adjoint_kernel<T, N, D, P>;
+    auto kernel = gmats != nullptr ? kronblockadj::kron_block_adjoint_kernel<T, N, D, P, true>
+                                   : kronblockadj::kron_block_adjoint_kernel<T, N, D, P, false>;
     long const cus = device_cu_count();
     long const grid = (std::min<long>(s.nb, cus * resident_per_cu(kernel, P, 0)) + 7) / 8 * 8;
     long const shared = (cus * kBlockAdjointSharedPerCu + 7) / 8 * 8;

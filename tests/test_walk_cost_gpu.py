@@ -10,7 +10,7 @@ from kronmult993_amd.device import DeviceBatch
 pytestmark = pytest.mark.gpu
 
 
-def _input_gradient_us(d, n, nb, inputs, dtype):
+def _input_gradient_us(d, n, nb, inputs, dtype, intermediates="auto"):
     """Fastest of seven replays of ten calls: entry k has input k % inputs."""
     size, k = n ** d, np.arange(nb)
     rng = np.random.default_rng(nb + inputs)
@@ -19,7 +19,7 @@ def _input_gradient_us(d, n, nb, inputs, dtype):
     b = W.HostBatch(f"walk_d{d}n{n}_{nb}_{inputs}", d, n, n, m, off.reshape(-1), x, (k % inputs) * size, nb // 4 + 1,
                     k // 4, grad_out_pool=rng.standard_normal((nb // 4 + 1) * size)).astype(dtype)
     db = DeviceBatch(b)
-    db.adjoint_setup(want_mats=False)
+    db.adjoint_setup(want_mats=False, intermediates=intermediates)
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
         db.run_adjoint(sync=False, stream=s)
@@ -45,7 +45,7 @@ def test_looking_for_the_period_is_cheap(gpu, d, n, dtype):
     """Where a batch outgrows the resident workgroups they look for the period first. Half as many entries again cost
     at most half the time again, a second round of entries and one trip to memory: below 2.2 times in all (a search
     that is a chain of loads: 2.5 to 3.2 times)."""
-    sizes = (1400, 2100, 3100, 4400, 6300)
+    sizes = (1400, 2100, 3100, 4400, 6300, 9400, 14000, 20000)
     t = [_input_gradient_us(d, n, nb, nb, dtype) for nb in sizes]
     assert max(b / a for a, b in zip(t, t[1:])) < 2.2, t
 
