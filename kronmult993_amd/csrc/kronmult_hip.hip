@@ -1120,6 +1120,21 @@ hipError_t reg_terms_launch(Shape const &s, int nterm, T const *const *mats, T c
     return hipGetLastError();
 }
 
+// d = 6, n = 4 in FP32: a wavefront per entry (kron_wave_terms.hpp) or four (kron_reg.hpp). Measured, four per entry / one,
+// us, 64 entries per output and (in brackets) one:
+//   16 entries, 3 terms 7.6 / 10.9 (7.5 / 11.8); 300, 2 terms 11.2 / 9.7 (9.4 / 11.9); 260, 3 terms 11.5 / 11.5 (10.4 /
+//   13.5); 400, 5 terms 16.1 / 16.1 (14.8 / 19.5); 1024, 3 terms 20.9 / 14.0 (20.0 / 23.2): from one entry per CU on, 1.5
+//   with more than two terms;
+//   2300, 2 terms 24.7 / 23.5 (35.5 / 45.8), 3 terms 31.0 / 31.3 (39.7 / 51.6); 3000, 3 terms 37.3 / 31.3 (49.6 / 53.1); 8192,
+//   3 terms 84.7 / 57.4 (121 / 121): not just above 8 entries per CU, where half of the wavefronts would take two.
+// Where no two entries share an output the atomics decide and one wavefront's longer chain shows; nothing on the host
+// says whether they do, and the operators that have several terms do share theirs.
+bool terms_by_wave(int nb, int nterm)
+{
+    long const cus = device_cu_count(), full = cus * kronwaveterms::kWavesPerCu;
+    return (nterm > 2 ? 2l * nb > 3 * cus : nb > cus) && !(nterm > 1 && nb > full && nb <= full + 2 * cus);
+}
+
 // The fused kernel where a register-resident plan exists, else one launch of the one-term path per term
 // (term t's factor pointers start at mats + t*nb*d).
 template<typename T>
@@ -1134,7 +1149,7 @@ hipError_t terms_launch(int d, int n, int nterm, T const *const *mats, int strid
     if (mats == nullptr || in == nullptr || out == nullptr) return hipErrorInvalidValue;
     T const *const *cin = reinterpret_cast<T const *const *>(in);
     if constexpr (sizeof(T) == 4)
-        if (s.d == 6 && s.n == 4)
+        if (s.d == 6 && s.n == 4 && terms_by_wave(nb, nterm))
         {
             Launch L;
             return wave_terms_launch(s, nterm, L, mats, cin, out, stream, true);
