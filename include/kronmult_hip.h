@@ -252,8 +252,10 @@ long long kronmult_batched_adjoint_workspace(int matrix_count, int matrix_size, 
  *                                a quarter of the tile per wavefront, by default 4 entries, 2 above 64 elements);
  *                                any other group gets a launch of its own, as below;
  *   KRONMULT_GROUPED_SEPARATE    one ordinary launch per group, shaped by that group's `tuning`;
- *   KRONMULT_GROUPED_AUTO        the persistent strategy, with launches of their own for large groups that a
- *                                single-batch kernel sweeps faster.
+ *   KRONMULT_GROUPED_AUTO        the persistent strategy, with launches of their own, in the library's default
+ *                                shape, for groups of 2^20 elements and more that a single-batch kernel sweeps
+ *                                faster; a group with `entries_per_tile`, and every group when
+ *                                `workgroups_per_cu` is given, stays in the persistent launch.
  * Only the first 16 groups can take part in the persistent launch; later groups get launches of their own.
  */
 #define KRONMULT_GROUPED_AUTO 0

@@ -1501,9 +1501,16 @@ hipError_t kronmult_grouped_launch(GroupT const *groups, int count, kronmult_gro
     kronmult_grouped_options_t const opt = options ? *options : kronmult_grouped_options_t{0, 0};
     if (opt.strategy < KRONMULT_GROUPED_AUTO || opt.strategy > KRONMULT_GROUPED_SEPARATE || opt.workgroups_per_cu < 0)
         return hipErrorInvalidValue;
+    // A group that AUTO gives a launch of its own takes the library's default shape; one with a hint for the persistent
+    // launch (its tile, the grid) stays in it.
+    kronmult_tuning_t const defaults{0, 0, 0};
+    auto own_launch = [&](GroupT const &g, Shape const &s) {
+        return opt.strategy == KRONMULT_GROUPED_AUTO && opt.workgroups_per_cu == 0 && g.entries_per_tile == 0 &&
+               group_own_launch<T>(s);
+    };
     // validate everything before launching anything
     Shape shapes[krongroup::kMaxGroups];
-    bool persistent[krongroup::kMaxGroups];
+    bool persistent[krongroup::kMaxGroups], by_auto[krongroup::kMaxGroups];
     int n_persistent = 0;
     for (int i = 0; i < count; ++i)
     {
@@ -1516,18 +1523,19 @@ hipError_t kronmult_grouped_launch(GroupT const *groups, int count, kronmult_gro
                                g.output_batched == nullptr))
             return hipErrorInvalidValue;
         // groups past the first kMaxGroups always get launches of their own
-        bool const pers = opt.strategy != KRONMULT_GROUPED_SEPARATE && i < krongroup::kMaxGroups &&
-                          group_persistent_ok<T>(g, s) && g.nb_batch > 0 &&
-                          !(opt.strategy == KRONMULT_GROUPED_AUTO && group_own_launch<T>(s));
+        bool const fits = opt.strategy != KRONMULT_GROUPED_SEPARATE && i < krongroup::kMaxGroups &&
+                          group_persistent_ok<T>(g, s) && g.nb_batch > 0;
+        bool const chosen = fits && own_launch(g, s), pers = fits && !chosen;
         if (i < krongroup::kMaxGroups)
         {
             shapes[i] = s;
             persistent[i] = pers;
+            by_auto[i] = chosen;
         }
         if (!pers)
         {
             Launch L;
-            kronmult_tuning_t const tu = g.tuning;
+            kronmult_tuning_t const tu = chosen ? defaults : g.tuning;
             err = kronmult_launch<T>(g.matrix_count, g.matrix_size, g.matrix_list_batched, g.matrix_stride,
                                      g.input_batched, g.output_batched, g.workspace_batched, 0, &tu, nullptr, &L);
             if (err != hipSuccess) return err;
@@ -1543,7 +1551,8 @@ hipError_t kronmult_grouped_launch(GroupT const *groups, int count, kronmult_gro
         if (g.nb_batch == 0) continue;
         hipError_t err = kronmult_launch<T>(g.matrix_count, g.matrix_size, g.matrix_list_batched, g.matrix_stride,
                                             g.input_batched, g.output_batched, g.workspace_batched, g.nb_batch,
-                                            &g.tuning, stream, nullptr);
+                                            i < krongroup::kMaxGroups && by_auto[i] ? &defaults : &g.tuning, stream,
+                                            nullptr);
         if (err != hipSuccess) return err;
     }
     if (n_persistent == 0) return hipSuccess;
