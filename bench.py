@@ -299,7 +299,8 @@ def main() -> int:
         for db in dbs:
             db.reset_output()
         groups, structs, kw = grouped_call_from_choice(dbs, choice)
-        kernel = "group_persistent" if choice["strategy"] == "persistent" else "separate launches"
+        kernel = {"persistent": "group_persistent", "auto": "group_persistent + separate launches"}.get(
+            choice["strategy"], "separate launches")
         step = lambda s: api.kronmult_batched_grouped(groups, dtype=args.dtype, stream=s, structs=structs, **kw)
         extra_config = {"groups": [[hb.d, hb.n, hb.nb] for hb in batches], "autotuned": choice}
     log(f"[bench] {'+'.join(hb.name for hb in batches)} {args.dtype}: kernel={kernel} on "

@@ -7,13 +7,14 @@ is process-wide, guarded by a lock, and optionally persisted as JSON (path argum
 variable KRONMULT_TUNE_CACHE).
 
 Choices:
-  * one batch: the kernel family (register-resident sweep where a plan exists, matrix-core sweep for
-    d=6 n=4 FP64, packed fiber sweep for small vectors, fiber sweep) and, for the register, matrix-core and
-    packed families, workgroups per CU;
+  * one batch: the library's default, or a kernel family (register-resident sweep where a plan exists,
+    matrix-core sweep for d=6 n=4 FP64, packed fiber sweep and wavefront sweep for small vectors, fiber sweep)
+    and, for the register, matrix-core and packed families, workgroups per CU, for the wavefront sweep entries
+    per workgroup;
   * several batches (a grouped call): the persistent launch -- workgroups per CU and per-group tile length
     (entries per tile, from a quarter of the entries the launch processes in one pass, which also shrinks
-    the pass and its LDS, to four passes) -- against one launch per group with each group's own best
-    shape.
+    the pass and its LDS, to four passes), or its default shape -- against one launch per group with each
+    group's own best shape, and the automatic strategy.
 """
 from __future__ import annotations
 
@@ -31,6 +32,7 @@ _LOADED: set = set()
 
 LDS_BUDGET = 64 * 1024      # the persistent launch's LDS budget per workgroup (kron_group.hpp host side)
 GROUP_THREADS = 256
+OWN_LAUNCH_ELEMS = 1 << 20  # a group below this many elements stays in the persistent launch (same rule as the library)
 
 
 def _torch():
@@ -131,7 +133,8 @@ class Autotuner:
         hit = None if force else self.lookup(key)
         if hit is not None:
             return hit
-        cands = [{"family": api.FAMILY_FIBER}]
+        # what an untuned call runs comes first: some kernels are reached by no explicit request
+        cands = [{"family": api.FAMILY_AUTO}, {"family": api.FAMILY_FIBER}]
         try:
             api.launch_info(db.d, db.n, db.itemsize, db.nb, {"family": api.FAMILY_REGISTER})
             cands += [{"family": api.FAMILY_REGISTER, "workgroups_per_cu": w} for w in (1, 2, 4, 8, 16)]
@@ -145,7 +148,7 @@ class Autotuner:
         try:
             api.launch_info(db.d, db.n, db.itemsize, db.nb, {"family": api.FAMILY_WAVE})
             cands += [{"family": api.FAMILY_WAVE}] + [{"family": api.FAMILY_WAVE, "entries_per_workgroup": e}
-                                                      for e in (1, 2, 4)]
+                                                      for e in (1, 2, 4, 8, 16)]
         except api.KronmultError:
             pass
         try:
@@ -181,6 +184,15 @@ class Autotuner:
                 "tunings": tun_clean}
         best_t = self._time_us(lambda st: api.kronmult_batched_grouped(groups, dtype=dt, strategy="separate",
                                                                        stream=st, structs=structs))
+        # what an untuned call runs: the persistent launch in its default shape and, with a group that may take a
+        # launch of its own, the automatic strategy
+        for strategy in ("persistent", "auto")[:2 if any(db.nb * db.size >= OWN_LAUNCH_ELEMS for db in dbs) else 1]:
+            t = self._time_us(lambda st: api.kronmult_batched_grouped(groups, dtype=dt, strategy=strategy, stream=st,
+                                                                      structs=structs))
+            if t < (best_t if strategy == "persistent" else 0.98 * best_t):  # (the same launch with no such group)
+                best_t = t
+                best = {"strategy": strategy, "workgroups_per_cu": 0, "entries_per_tile": [0] * len(dbs),
+                        "tunings": tun_clean}
         # persistent launch: grid and tile length, the same multiple of each group's pass for all groups ...
         mults = (0.25, 0.5, 1, 2, 4)
         tile = lambda db, m: max(1, int(entries_per_pass(db.d, db.n, db.itemsize) * m))
