@@ -342,7 +342,10 @@ int kronmult_build_element_batch_f32(int matrix_count, int matrix_size, int base
 
 /*
  * Library version string and the name of the kernel the dispatcher would pick for (d, n, element size in
- * bytes, nb_batch); both point to static storage. No reference counterpart (diagnostics only).
+ * bytes, nb_batch); both point to static storage. No reference counterpart (diagnostics only). The name begins
+ * with the family ("wave", "packed", "reg_sweep", "wide_lds", "wide_global"; in the fiber family "fiber_lds",
+ * "fiber_global" and "multipass", the last two with a workspace); several kernels may share a name, the launch
+ * information above tells them apart.
  */
 char const *kronmult_hip_version(void);
 char const *kronmult_hip_kernel_name(int matrix_count, int matrix_size, int element_size, int nb_batch);

@@ -360,6 +360,18 @@ hipError_t wave_terms_launch(Shape const &s, int nterm, Launch &L, float const *
     return hipGetLastError();
 }
 
+// One term of d = 6, n = 4 in FP32: a wavefront per entry where every wavefront has one entry and there is one for every
+// CU (500 entries 9.4 -> 7.2 us, 1024 15.7 -> 9.1, 2048 18.1 -> 13.7; with outputs of their own 300 entries 8.2 -> 9.8, 800
+// 14.5 -> 16.1, 1500 24.6 -> 24.8: the atomics decide there and the chain of one wavefront is longer). Below, four
+// wavefronts per entry finish sooner (130 entries 4.9 against 6.3 us); above, the sweep is bound by its input, which they
+// read ahead better (8192 entries 42.0 against 45.8 us).
+bool one_term_by_wave(Shape const &s, kronmult_tuning_t const &tu)
+{
+    long const cus = device_cu_count();
+    return !s.ordered && tu.entries_per_workgroup <= 0 && tu.workgroups_per_cu <= 0 && s.nb > cus &&
+           s.nb <= cus * kronwaveterms::kWavesPerCu;
+}
+
 template<typename T, int D, int N>
 hipError_t reg_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L, T const *const *mats,
                       T const *const *in, T *const *out, T *const *ws, hipStream_t stream, bool run)
@@ -367,16 +379,7 @@ hipError_t reg_launch(Shape const &s, kronmult_tuning_t const &tu, Launch &L, T 
     using PL = kronplan::Plan<D, N, reg_rho(D, N)>;
     static_assert(PL::P % 64 == 0 && PL::P <= 1024, "plan must fill whole wavefronts");
     if constexpr (sizeof(T) == 4 && D == 6 && N == 4)
-    {
-        // One term: a wavefront per entry where every wavefront has one entry and there is one for every CU (500 entries
-        // 9.4 -> 7.2 us, 1024 15.7 -> 9.1, 2048 18.1 -> 13.7). Below, four wavefronts per entry finish sooner (130
-        // entries 4.9 against 6.3 us); above, the sweep is bound by its input, which they read ahead better (8192
-        // entries 42.0 against 45.8 us).
-        long const cus = device_cu_count();
-        if (!s.ordered && tu.entries_per_workgroup <= 0 && tu.workgroups_per_cu <= 0 && s.nb > cus &&
-            s.nb <= cus * kronwaveterms::kWavesPerCu)
-            return wave_terms_launch(s, 1, L, mats, in, out, stream, run);
-    }
+        if (one_term_by_wave(s, tu)) return wave_terms_launch(s, 1, L, mats, in, out, stream, run);
     auto kernel = s.ordered ? kronreg::kron_reg_kernel<T, PL, true> : kronreg::kron_reg_kernel<T, PL, false>;
     L.lds = sizeof(T) * (PL::SIZE + (kronreg::fwd_coef_in_lds<T, PL>() ? kronreg::Coef<T, PL>::kCount : 0));
     if constexpr (m8_plan<T>(D, N))
@@ -819,13 +822,19 @@ hipError_t block_passes(Shape const &s, Launch &L, T const *const *mats, T const
     return hipErrorInvalidValue;
 }
 
+// shapes of the fiber family that the whole-fiber wavefront kernel sweeps
+bool fiber_by_wave(Shape const &s)
+{
+    return (s.d == 3 && (s.n == 6 || s.n == 7)) || (s.d == 4 && s.n == 5);
+}
+
 template<typename T>
 hipError_t fiber_dispatch(Shape const &s, Launch &L, T const *const *mats, T const *const *in, T *const *out,
                           T *const *ws, hipStream_t stream, bool run)
 {
     if (s.n > kMaxFiber) return wide_dispatch<T>(s, L, mats, in, out, ws, stream, run);
     // (4,3), (5,3), (7,2) and (8,2) come here only when a caller asks for this family: the general kernel
-    if (!s.ordered && ((s.d == 3 && (s.n == 6 || s.n == 7)) || (s.d == 4 && s.n == 5)))
+    if (!s.ordered && fiber_by_wave(s))
         return wave_fiber_launch<T>(s, KRONMULT_FAMILY_FIBER, 0, L, mats, in, out, stream, run);
     bool const block = !s.ordered && kronblock::block_shape<T>(s.d, s.n);
     if (fiber_in_lds<T>(s))
@@ -1179,6 +1188,8 @@ int kronmult_sync(int d, int n, T const *const *mats, int stride, T **in, T **ou
     return static_cast<int>(hipDeviceSynchronize());
 }
 
+// The names begin with the family and, in the fiber family, with where the vector lives; "_block", "_wave" and "mfma" tell
+// the kernel where a family has several. (A shape of the whole-fiber kernel has one kernel under three families' names.)
 template<typename T>
 char const *kernel_name(int d, int n, int nb)
 {
@@ -1192,6 +1203,7 @@ char const *kernel_name(int d, int n, int nb)
     case KRONMULT_FAMILY_WAVE: return f64 ? "wave_f64" : "wave_f32";
     case KRONMULT_FAMILY_REGISTER:
         if (m8_plan<T>(s.d, s.n)) return "reg_sweep_mfma_f64";
+        if (!f64 && s.d == 6 && s.n == 4 && one_term_by_wave(s, kronmult_tuning_t{0, 0, 0})) return "reg_sweep_wave_f32";
         return f64 ? "reg_sweep_f64" : "reg_sweep_f32";
     case KRONMULT_FAMILY_FIBER:
         if (s.n > kMaxFiber)
@@ -1202,8 +1214,14 @@ char const *kernel_name(int d, int n, int nb)
             if (in_lds) return f64 ? "wide_lds_f64" : "wide_lds_f32";
             return f64 ? "wide_global_f64" : "wide_global_f32";
         }
+        if (fiber_by_wave(s)) return f64 ? "fiber_lds_wave_f64" : "fiber_lds_wave_f32";
+        if (kronblock::block_shape<T>(s.d, s.n))
+        {
+            if (fiber_in_lds<T>(s)) return f64 ? "fiber_lds_block_f64" : "fiber_lds_block_f32";
+            return f64 ? "fiber_global_block_f64" : "fiber_global_block_f32";  // (asks for a workspace)
+        }
         if (fiber_in_lds<T>(s)) return f64 ? "fiber_lds_f64" : "fiber_lds_f32";
-        if (use_passes<T>(s)) return f64 ? "multipass_f64" : "multipass_f32";
+        if (kronblock::pass_shape<T>(s.d, s.n) || use_passes<T>(s)) return f64 ? "multipass_f64" : "multipass_f32";
         return f64 ? "fiber_global_f64" : "fiber_global_f32";
     default: return "unsupported";
     }
