@@ -20,7 +20,6 @@
 
 #include <cstdint>
 #include <type_traits>
-#include <type_traits>
 
 #include "kron_plan.hpp"
 #include "kron_runs.hpp"
@@ -794,7 +793,7 @@ __global__ void __launch_bounds__(PL::P) __attribute__((amdgpu_waves_per_eu(min_
             Lds<T, PL>::template read<0>(lds, v, t);
             run_phases<T, PL, 0, true>(lds, v, mats + static_cast<size_t>(e) * PL::kD, stride, coef, t);
             if constexpr (!kCoefLds) flush_if_new(e);
-    #pragma unroll
+#pragma unroll
             for (int j = 0; j < PL::R; ++j) acc[j] += v[j];
         }
         if constexpr (ORDERED)
