@@ -1,4 +1,4 @@
-// kron_block.hpp -- contiguous blocks of a vector swept in LDS: whole entries of 4 KB to 80 KB, and the fastest modes
+// kron_block.hpp -- contiguous blocks of a vector swept in LDS: whole entries of 3 KB to 80 KB, and the fastest modes
 // of larger ones (kron_final.hpp applies the two that are left).
 //
 // A block is Q consecutive sub-tensors of n^G elements. The workgroup stages it in LDS and contracts its G modes in

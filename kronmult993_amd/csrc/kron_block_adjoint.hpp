@@ -16,10 +16,11 @@
 // What bounds it: the chain of an entry (2 d LDS exchanges, d reduce-scatters, about 900 instructions for d=4 n=4), then
 // the input gradient's atomics. The general kernel (kron_adjoint.hpp) rebuilds X_t for every t, takes the products on
 // matrix instructions with n of 16 rows in use (FP32), and adds every entry's gradients with atomics of their own. 8192
-// entries, FP64 / FP32, general kernel -> here: d=4 n=5 with inputs of their own and 256 factor sets 191 -> 74 / 104 ->
-// 42 us, as 128 x 64 element pairs 192 -> 77 / 204 -> 61; d=5 n=5 1159 -> 854 / 618 -> 238 (FP64 spills: 10 wavefronts
-// leave it 168 registers); d=4 n=6 313 -> 244 / 189 -> 103; d=6 n=3 169 -> 90 / 260 -> 55; d=3 n=7 pairs 124 -> 84 / 243
-// -> 72; against the register kernel d=5 n=4 110 -> 97 / 61 -> 53, d=4 n=8 FP32 328 -> 283.
+// entries, FP64 / FP32, general kernel -> here: d=4 n=5 with inputs of their own and 256 factor sets 191 -> 72 / 104 ->
+// 37 us, as 128 x 64 element pairs 193 -> 75 / 198 -> 56; d=5 n=5 1159 -> 422 / 618 -> 237 (10 wavefronts leave it 168
+// registers; the scalar factor columns spill); d=4 n=6 313 -> 248 / 189 -> 96; d=6 n=3 169 -> 87 / 260 -> 51; d=3 n=7
+// pairs 125 -> 72 / 243 -> 61; against the register kernel d=5 n=4 110 -> 95 / 61 -> 53, d=4 n=8 FP32 328 -> 274. The
+// input gradient alone, inputs of their own, 1100 entries: d=5 n=5 FP64 36.8 -> 29.8, 700 of d=4 n=7 FP32 13.4 -> 11.1.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -415,9 +416,10 @@ __global__ void __launch_bounds__(P)
     flush();
 }
 
-// The shapes, as X(D, N). FP64 leaves d=3 n=5, d=3 n=6 and d=4 n=3 to the general kernel (8192 entries with inputs of their
-// own 37, 50, 27 us here against 36, 45, 22; shared factors 66, 67, 49 against 124, 131, 66) and d=4 n=8 to the register
-// kernel (484 against 501, 300 entries 36 against 34).
+// The shapes, as X(D, N). FP64 leaves d=3 n=5, d=3 n=6 and d=4 n=3 to the general kernel and d=4 n=8 to the register
+// kernel: the line was drawn when the walk's search for the period took about 10 us of every call (8192 entries with
+// inputs of their own 37, 50, 27 us here against 36, 45, 22; d=4 n=8 300 entries 36 against 34). Without it they take
+// 26, 40, 18 us here, and d=4 n=8 477 against 501 (300 entries 35 against 34).
 #define KRON_BLOCK_ADJOINT_SHAPES(X)                                                                                \
     X(3, 5) X(3, 6) X(3, 7) X(4, 3) X(4, 5) X(4, 6) X(4, 7) X(4, 8) X(5, 3) X(5, 4) X(5, 5) X(6, 2) X(6, 3)
 

@@ -18,8 +18,8 @@
 //
 // What bounds it: latency, with two wavefronts per SIMD (64 input values, 64 working values and 64 sums per lane); the
 // matrix cores take 36 us of 24576 sweeps at their measured 135 TFLOP/s. Measured against 256 threads per entry: 8192
-// entries of a 128 x 64 operator, 3 terms 70.6 -> 56.1 us, 2 terms 52.9 -> 41.5; 2048 entries, 3 terms 28.6 -> 22.2;
-// 16 entries 13.0 -> 12.7.
+// entries of a 128 x 64 operator, 3 terms 70.6 -> 56.1 us, 2 terms 52.9 -> 41.5; 2048 entries, 3 terms 28.6 -> 22.2.
+// Few entries, and outputs that are not shared, are faster with 256 threads (figures at the dispatch).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1346,7 +1346,7 @@ hipError_t reg_adjoint_launch(Shape const &s, RegAdjMode mode, T const *const *m
 }
 
 // d = 6, n = 4: the two-modes-per-phase adjoint (kron_reg_adjoint2.hpp), one run per resident workgroup.
-// It serves AUTO (measured on the d=6 batch, listed by output: FP64 189 us, FP32 112 us, against 522 / 304 us for the
+// It serves AUTO (measured on the d=6 batch, listed by output: FP64 172 us, FP32 101 us, against 522 / 304 us for the
 // one-mode-per-phase kernel, which RECOMPUTE and STORE keep).
 // At most three workgroups per CU: the input gradient alone would leave room for six in FP32, whose shorter runs sum less
 // (as 64-input pairs, 3 / 6 per CU: 2100 entries 17.6 / 25.7 us, 8300 39.5 / 36.3).
@@ -1368,7 +1368,7 @@ hipError_t adjoint2_launch(Shape const &s, T const *const *mats, T const *const 
 // Whole entries on the block layout (kron_block_adjoint.hpp), AUTO: every resident workgroup takes an equal part of the
 // entries; where the entries share factor gradients (looked for on the device) only this many per CU do, whose longer
 // runs make fewer atomic adds to the same few addresses. Measured, 128 x 64 element pairs FP32, at 2 / 4 / 8 / all: d=4 n=5
-// 71 / 61 / 75 / 76 us, d=6 n=2 50 / 42 / 48 / 69, d=3 n=7 85 / 71 / 82 / 83.
+// 69 / 56 / 70 / 70 us, d=6 n=2 40 / 32 / 38 / 86, d=3 n=7 76 / 61 / 73 / 91.
 constexpr long kBlockAdjointSharedPerCu = 4;
 
 template<typename T, int D, int N>
