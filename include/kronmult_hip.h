@@ -55,9 +55,11 @@ int kronmult_batched_f32_async(int matrix_count, int matrix_size, float const *c
  *   family:                 KRONMULT_FAMILY_AUTO, _REGISTER (register-resident sweep, only for the
  *                           (d, n) plans it is built for), _FIBER (fiber sweep, one vector per
  *                           workgroup, any n with n * sizeof(T) <= 32 KiB; n > 64 on the wide-fiber
- *                           kernel), _MATRIX (every contraction on the FP64 matrix cores;
+ *                           kernel; the block sweep, two passes, or whole fibers per lane for the shapes
+ *                           these are built for), _MATRIX (every contraction on the FP64 matrix cores;
  *                           d = 6, n = 4, double only) or _PACKED (fiber sweep with several small vectors per workgroup: n <= 8,
- *                           n^(d-1) <= 64; the default for such shapes from 20 entries per CU on) or
+ *                           n^(d-1) <= 64; the default for such shapes from 20 entries per CU on; with
+ *                           both of the fields below left at 0, whole fibers per lane where that is built) or
  *                           _WAVE (one wavefront per entry: n^d <= 64 with 2 <= n <= 8, one element per lane,
  *                           and d=3 n=5; d=2 n=9,10 with two, and d=7,8 n=2; d=4,5 n=3; d=3 n=6 with
  *                           whole fibers per lane: there a workgroup is four wavefronts, which take a quarter of
